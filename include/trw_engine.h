@@ -253,8 +253,8 @@ trw_status trw_sample_device(void* handle, const trw_sample_params* params, trw_
  * max_walk_len - 1 and (max_walk_len - 1) * feature_dim values); on return
  * num_walks, max_walk_len and feature_dim are set.  Every per-call buffer
  * (start keys and states, draws, processing order, walk scratch) comes from a
- * fixed device array of 128 MiB per device, held until the process ends: a
- * sample needing more (about 40 B per walk, plus 8 B per slot of walk scratch
+ * fixed device array of 128 MiB per device (and 2 MiB of sort scratch beside
+ * it), held until the process ends: a sample needing more (about 40 B per walk, plus 8 B per slot of walk scratch
  * -- 640 B per walk at max_walk_len 80 -- where a layout pass writes the
  * rows), more walks than capacity_walks, or misaligned buffers, is rejected
  * with TRW_ERR_INVALID_ARGUMENT.  Calls on one

@@ -1277,8 +1277,7 @@ void build_direction(Engine& e, DirIndex& dir, size_t n, int key_bits, size_t vc
     e.k32b.ensure(n);
     e.k64a.ensure(n);
     if (packed) e.k64b.ensure(n);
-    e.hist.ensure(radix_hist_elems(n));
-    const int passes = n > 1 ? radix_passes(0, key_bits) : 0;
+    const int passes = radix_passes(n, 0, key_bits);
     // unpacked, the sorted records land in dir.rec: start in the buffer set
     // the last digit pass does not write into
     uint64_t* recs = reinterpret_cast<uint64_t*>(dir.rec.p);
@@ -1289,7 +1288,8 @@ void build_direction(Engine& e, DirIndex& dir, size_t n, int key_bits, size_t vc
         hipLaunchKernelGGL(node_entries_kernel, dim3(grid_for(edges)), dim3(kB), 0, s, e.src.p,
                            e.dst.p, edges, mode, 0u, packed ? e.erank.p : nullptr, nb, eb,
                            e.k32a.p, v0);
-    const int which = radix_sort_u32_v64(e.k32a.p, v0, e.k32b.p, v1, n, 0, key_bits, e.hist.p, s);
+    const int which = radix_sort_u32_v64(e.k32a.p, v0, e.k32b.p, v1, n, 0, key_bits,
+                                         e.radix_tmp(n, key_bits), s);
     // the sorted keys become the direction's (the scratch takes the old
     // buffer, which every user sizes again before writing)
     dir.key.swap(which ? e.k32b : e.k32a);
@@ -1324,14 +1324,13 @@ void append_direction(Engine& e, DirIndex& dir, int mode, int key_bits, size_t v
     e.k32b.ensure(m);
     e.k64a.ensure(m);
     e.k64b.ensure(m);
-    e.hist.ensure(radix_hist_elems(m));
     const uint32_t id0 = static_cast<uint32_t>(e.append_kept_old);
     if (e.append_kept_new)
         hipLaunchKernelGGL(node_entries_kernel, dim3(grid_for(e.append_kept_new)), dim3(kB), 0, s,
                            e.src.p + id0, e.dst.p + id0, e.append_kept_new, mode, id0, nullptr, 0,
                            0, e.k32a.p, e.k64a.p);
     const int w = radix_sort_u32_v64(e.k32a.p, e.k64a.p, e.k32b.p, e.k64b.p, m, 0, key_bits,
-                                     e.hist.p, s);
+                                     e.radix_tmp(m, key_bits), s);
     const uint32_t* bkeys = w ? e.k32b.p : e.k32a.p;
     const uint64_t* brec = w ? e.k64b.p : e.k64a.p;
     e.inc_bstart.resize(vc);
@@ -1562,7 +1561,7 @@ SortedBatch sort_batch(Engine& e, const int32_t* d_src, const int32_t* d_dst, co
     if (carry_ends) e.ends64b.ensure(n);
     e.v32a.ensure(n);
     e.v32b.ensure(n);
-    e.hist.ensure(radix_hist_elems(n));
+    const RadixTmp tmp = e.radix_tmp(n, bits);
     uint32_t* k32s[2] = {reinterpret_cast<uint32_t*>(e.k64a.p), reinterpret_cast<uint32_t*>(e.k64b.p)};
     uint32_t* pos0 = carry_ends ? nullptr : e.v32a.p;
     int which;
@@ -1571,17 +1570,17 @@ SortedBatch sort_batch(Engine& e, const int32_t* d_src, const int32_t* d_dst, co
                            e.ts.p, e.src.p, e.dst.p, size_t{0}, d_ts, d_src, d_dst, n, btmin,
                            k32s[0], pos0, e.ends64.p);
         which = carry_ends ? radix_sort_u32_v64(k32s[0], e.ends64.p, k32s[1], e.ends64b.p, n, 0,
-                                                bits, e.hist.p, s)
+                                                bits, tmp, s)
                            : radix_sort_u32(k32s[0], e.v32a.p, k32s[1], e.v32b.p, n, 0, bits,
-                                            e.hist.p, s);
+                                            tmp, s);
     } else {
         hipLaunchKernelGGL((make_ts_keys_kernel<uint64_t>), dim3(grid_for(n)), dim3(kB), 0, s,
                            e.ts.p, e.src.p, e.dst.p, size_t{0}, d_ts, d_src, d_dst, n, btmin,
                            e.k64a.p, pos0, e.ends64.p);
         which = carry_ends ? radix_sort_u64_v64(e.k64a.p, e.ends64.p, e.k64b.p, e.ends64b.p, n, 0,
-                                                bits, e.hist.p, s)
+                                                bits, tmp, s)
                            : radix_sort_u64(e.k64a.p, e.v32a.p, e.k64b.p, e.v32b.p, n, 0, bits,
-                                            e.hist.p, s);
+                                            tmp, s);
     }
     SortedBatch b;
     b.keys32 = keys32;
@@ -1664,7 +1663,10 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
     if (carry_ends) ends64b.ensure(etot);
     v32a.ensure(std::max(etot, 2 * etot));
     v32b.ensure(std::max(etot, 2 * etot));
-    hist.ensure(radix_hist_elems(2 * etot));
+    // (sized for the node index's sorts as well, so that it grows once)
+    const int id_bits = std::max(1, bit_length_u64(static_cast<uint64_t>(batch_max_id)));
+    hist.ensure(radix_tmp_elems(cfg.is_directed ? etot : 2 * etot, id_bits));
+    const RadixTmp tmp = radix_tmp(etot, bits);
     uint32_t* k32s[2] = {reinterpret_cast<uint32_t*>(k64a.p), reinterpret_cast<uint32_t*>(k64b.p)};
     uint32_t* pos0 = carry_ends ? nullptr : v32a.p;
     // the window's cut (step 3), known before the sort: when it keeps every
@@ -1691,12 +1693,12 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
                            ends64.p);
         if (fold)
             folded = radix_sort_u32_v64_store(k32s[0], ends64.p, k32s[1], ends64b.p, etot, 0, bits,
-                                              hist.p, s, st);
+                                              tmp, s, st);
         else
             which = carry_ends
                         ? radix_sort_u32_v64(k32s[0], ends64.p, k32s[1], ends64b.p, etot, 0, bits,
-                                             hist.p, s)
-                        : radix_sort_u32(k32s[0], v32a.p, k32s[1], v32b.p, etot, 0, bits, hist.p,
+                                             tmp, s)
+                        : radix_sort_u32(k32s[0], v32a.p, k32s[1], v32b.p, etot, 0, bits, tmp,
                                          s);
     } else {
         hipLaunchKernelGGL((make_ts_keys_kernel<uint64_t>), dim3(grid_for(etot)), dim3(kB), 0, s,
@@ -1704,12 +1706,12 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
                            ends64.p);
         if (fold)
             folded = radix_sort_u64_v64_store(k64a.p, ends64.p, k64b.p, ends64b.p, etot, 0, bits,
-                                              hist.p, s, st);
+                                              tmp, s, st);
         else
             which = carry_ends
                         ? radix_sort_u64_v64(k64a.p, ends64.p, k64b.p, ends64b.p, etot, 0, bits,
-                                             hist.p, s)
-                        : radix_sort_u64(k64a.p, v32a.p, k64b.p, v32b.p, etot, 0, bits, hist.p, s);
+                                             tmp, s)
+                        : radix_sort_u64(k64a.p, v32a.p, k64b.p, v32b.p, etot, 0, bits, tmp, s);
     }
     uint32_t* perm = which ? v32b.p : v32a.p;
     const uint64_t* sorted_ends = which ? ends64b.p : ends64.p;
@@ -2118,7 +2120,6 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
         std::memcpy(&n_active, hs, 4);
         const int rb = std::max(1, bit_length_u64(n_active ? n_active - 1 : 0));
         const bool ranked = 2 * rb <= 32;
-        hist.ensure(radix_hist_elems(m2));
         const uint32_t* rkeys = nullptr;
         const uint64_t* fkeys = nullptr;
         if (ranked) {
@@ -2133,7 +2134,8 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
             if (E)
                 hipLaunchKernelGGL(adj_rank_keys_kernel, dim3(grid_for(E)), dim3(kB), 0, s, src.p,
                                    dst.p, E, adj_rank.p, rb, k32a.p);
-            const int w = radix_sort_u32(k32a.p, nullptr, k32b.p, nullptr, m2, 0, 2 * rb, hist.p, s);
+            const int w = radix_sort_u32(k32a.p, nullptr, k32b.p, nullptr, m2, 0, 2 * rb,
+                                         radix_tmp(m2, 2 * rb), s);
             rkeys = w ? k32b.p : k32a.p;
         } else {
             k64a.ensure(m2);
@@ -2141,7 +2143,8 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
             if (E)
                 hipLaunchKernelGGL(adj_pair_keys_kernel, dim3(grid_for(E)), dim3(kB), 0, s, src.p,
                                    dst.p, E, b, k64a.p);
-            const int w = radix_sort_u64(k64a.p, nullptr, k64b.p, nullptr, m2, 0, 2 * b, hist.p, s);
+            const int w = radix_sort_u64(k64a.p, nullptr, k64b.p, nullptr, m2, 0, 2 * b,
+                                 radix_tmp(m2, 2 * b), s);
             fkeys = w ? k64b.p : k64a.p;
         }
         // a set at most half full of the distinct pairs
@@ -2220,11 +2223,11 @@ void Engine::build_adjacency_lists() {
     const size_t m2 = 2 * E, v = adj_nodes;
     k64a.ensure(m2);
     k64b.ensure(m2);
-    hist.ensure(radix_hist_elems(m2));
     if (E)
         hipLaunchKernelGGL(adj_keys_kernel, dim3(grid_for(E)), dim3(kB), 0, s, src.p, dst.p, E, b,
                            k64a.p);
-    const int w = radix_sort_u64(k64a.p, nullptr, k64b.p, nullptr, m2, 0, 2 * b, hist.p, s);
+    const int w = radix_sort_u64(k64a.p, nullptr, k64b.p, nullptr, m2, 0, 2 * b,
+                                 radix_tmp(m2, 2 * b), s);
     uint64_t* ak = w ? k64b.p : k64a.p;
     adj_nbr.resize(m2);
     if (m2)

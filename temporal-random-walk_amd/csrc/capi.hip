@@ -306,6 +306,8 @@ trw_status trw_sample_device_noalloc(void* handle, const trw_sample_params* para
         trw::SampleTarget t{};
         t.space.base = static_cast<unsigned char*>(trw::noalloc_scratch(e.device));
         t.space.cap = trw::kNoAllocScratchBytes;
+        t.space.sort = reinterpret_cast<uint32_t*>(t.space.base + trw::kNoAllocScratchBytes);
+        t.space.sort_words = trw::kNoAllocSortBytes / sizeof(uint32_t);
         t.capacity_walks = capacity_walks;
         t.nodes = out->nodes;
         t.ts = out->timestamps;

@@ -138,6 +138,10 @@ struct DBuf {
 struct SampleSpace {
     unsigned char* base = nullptr;  // nullptr: the engine's buffers
     size_t cap = 0, used = 0;
+    // the region's own sort scratch, shared by the call's sorts (sorts that
+    // need more take theirs from the region)
+    uint32_t* sort = nullptr;
+    size_t sort_words = 0;
 
     // n elements: the engine buffer `own` (grown if needed) or the next
     // 256-byte aligned piece of the region
@@ -155,11 +159,20 @@ struct SampleSpace {
         used = off + n * sizeof(T);
         return reinterpret_cast<T*>(base + off);
     }
+    // scratch of a radix sort of n keys of `bits` bits
+    RadixTmp sort_tmp(DBuf<uint32_t>& own, size_t n, int bits) {
+        const size_t want = radix_tmp_elems(n, bits);
+        if (base && want <= sort_words) return RadixTmp{sort, sort_words};
+        const size_t words = base ? radix_min_elems(n, bits) : want;
+        return RadixTmp{take(own, words), words};
+    }
 };
 
 // Size of the device array trw_sample_device_noalloc takes its per-call
 // buffers from (one per device, held for the life of the process).
 constexpr size_t kNoAllocScratchBytes = size_t{128} << 20;
+// Its sort scratch beside that (SampleSpace::sort).
+constexpr size_t kNoAllocSortBytes = size_t{2} << 20;
 
 // Caller-owned device outputs of trw_sample_device_noalloc, and the fixed
 // scratch region its per-call buffers come from.
@@ -319,7 +332,11 @@ struct Engine {
     DBuf<uint64_t> k64a, k64b;
     DBuf<uint64_t> ends64, ends64b;  // packed (src, dst) of the timestamp sort's input
     DBuf<uint32_t> k32a, k32b, v32a, v32b;
-    DBuf<uint32_t> hist, flags, scan, scan_scratch;
+    DBuf<uint32_t> hist, flags, scan, scan_scratch;  // hist: radix sort scratch
+    RadixTmp radix_tmp(size_t n, int bits) {
+        hist.ensure(radix_tmp_elems(n, bits));
+        return RadixTmp{hist.p, hist.cap};
+    }
     DBuf<uint64_t> scan64_scratch;
     DBuf<double> dscratch, fscan_scratch;
     DBuf<double> gsum;         // the global weights' sums (side stream)

@@ -1,11 +1,11 @@
 // primitives.h -- device-wide scan and stable radix sort for the index build.
 //
 // Hand-written for CDNA4 (wave64): no rocPRIM / hipCUB.  The radix sort is a
-// classic LSD sort with four launches per digit pass (tile histograms; the
-// digit totals, one workgroup per digit summing its histogram row; one
-// workgroup per digit scanning that row; stable scatter); a sort of B key
-// bits takes the fewest passes of at most 10-bit
-// digits, the bits split evenly.  Stable ranking inside a tile uses wave-level
+// classic LSD sort with three launches per digit pass (tile histograms; one
+// workgroup per digit scanning its histogram row; stable scatter), or one launch
+// in all for inputs of one tile; a sort of B key bits takes the fewest passes
+// of at most 8-bit digits (10-bit where launches outweigh the data), the bits
+// split evenly.  Stable ranking inside a tile uses wave-level
 // multisplit: one 64-lane ballot per digit bit gives every lane the mask of
 // lanes holding the same digit, so the in-row rank is a popcount and a single
 // leader lane per digit bumps the wave's LDS counter.  Waves own
@@ -44,20 +44,26 @@ void running_max_f64(double* data, size_t n, double* scratch, hipStream_t s);
 // Stable sort of (key, value) pairs by key bits [begin_bit, end_bit).  Values
 // may be null (keys only).  Buffers are ping-ponged; the function returns 0 if
 // the sorted result ended in (keys0, vals0) and 1 if in (keys1, vals1).
-// `hist` must hold radix_hist_elems(n) uint32.
-size_t radix_hist_elems(size_t n);
+// tmp: device scratch; radix_tmp_elems(n, end_bit - begin_bit) words let every
+// size run its fastest form, radix_min_elems words let it run.
+struct RadixTmp {
+    uint32_t* p;
+    size_t n;  // words
+};
+size_t radix_tmp_elems(size_t n, int bits);
+size_t radix_min_elems(size_t n, int bits);
 int radix_sort_u64(uint64_t* keys0, uint32_t* vals0, uint64_t* keys1, uint32_t* vals1, size_t n,
-                   int begin_bit, int end_bit, uint32_t* hist, hipStream_t s);
+                   int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s);
 int radix_sort_u32(uint32_t* keys0, uint32_t* vals0, uint32_t* keys1, uint32_t* vals1, size_t n,
-                   int begin_bit, int end_bit, uint32_t* hist, hipStream_t s);
+                   int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s);
 // 64- and 32-bit keys with 64-bit values (a record carried through the sort).
 int radix_sort_u64_v64(uint64_t* keys0, uint64_t* vals0, uint64_t* keys1, uint64_t* vals1,
-                       size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s);
+                       size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s);
 int radix_sort_u32_v64(uint32_t* keys0, uint64_t* vals0, uint32_t* keys1, uint64_t* vals1,
-                       size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s);
-// Digit passes of a sort of bits [begin_bit, end_bit): the result lands in
-// buffer set (passes % 2) when n > 1.
-int radix_passes(int begin_bit, int end_bit);
+                       size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s);
+// Digit passes of a sort of n keys by bits [begin_bit, end_bit) with
+// radix_tmp_elems words of scratch: the result lands in buffer set (passes % 2).
+int radix_passes(size_t n, int begin_bit, int end_bit);
 
 // The edge store as the last pass of a sort of (timestamp key, packed
 // endpoints) writes it: src = low half, dst = high half of the value, ts =
@@ -73,10 +79,10 @@ struct SortedStore {
 // afterwards).  Returns false, writing nothing, when the sort has no pass
 // (n <= 1 or no key bits): the input is then already in order.
 bool radix_sort_u32_v64_store(uint32_t* keys0, uint64_t* vals0, uint32_t* keys1, uint64_t* vals1,
-                              size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s,
+                              size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
                               const SortedStore& out);
 bool radix_sort_u64_v64_store(uint64_t* keys0, uint64_t* vals0, uint64_t* keys1, uint64_t* vals1,
-                              size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s,
+                              size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
                               const SortedStore& out);
 
 // ---- reductions ---------------------------------------------------------------

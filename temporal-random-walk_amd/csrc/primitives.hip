@@ -2,6 +2,7 @@
 // See primitives.h for the design notes.
 #include "primitives.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #include <stdexcept>
@@ -36,7 +37,7 @@ struct OpMax {
 };
 
 // ---------------------------------------------------------------------------
-// block-level helpers (256 threads = 4 wave64)
+// block-level helpers (256 threads = 4 wave64, unless W says otherwise)
 // ---------------------------------------------------------------------------
 template <typename T, typename Op = OpSum>
 __device__ __forceinline__ T wave_inclusive_scan(T x, int lane) {
@@ -51,7 +52,7 @@ __device__ __forceinline__ T wave_inclusive_scan(T x, int lane) {
 // Exclusive block scan of one value per thread; *total receives the block
 // total.  The exclusive value is built from the wave prefix and the shifted
 // inclusive scan, so it is exact for the maximum as well as for integers.
-template <typename T, typename Op = OpSum>
+template <typename T, typename Op = OpSum, int W = kWaves>
 __device__ __forceinline__ T block_exclusive_scan(T v, T* total, T* s_wave) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const T inc = wave_inclusive_scan<T, Op>(v, lane);
@@ -60,7 +61,7 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* total, T* s_wave) {
     __syncthreads();
     T wp = Op::template identity<T>(), tot = Op::template identity<T>();
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
+    for (int w = 0; w < W; ++w) {
         const T sw = s_wave[w];
         if (w < wave) wp = Op::apply(wp, sw);
         tot = Op::apply(tot, sw);
@@ -245,19 +246,22 @@ void scan_impl(const T* in, T* out, size_t n, T* scratch, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// radix sort: a sort of B key bits takes the fewest passes of at most
-// kMaxDigitBits bits, the bits split evenly (27 bits: three 9-bit passes, 20
-// bits: two 10-bit passes); tile = 4 waves x 8 rows x 64 keys = 2048 keys; a
-// workgroup owns kTilesPerBlock consecutive tiles, so the digit-major
-// histogram has one column per workgroup (fewer scattered histogram writes and
-// a shorter histogram scan per pass)
+// radix sort: a sort of B key bits splits them evenly over its passes (27 bits:
+// four passes of 7).  The histogram kernel counts tiles of 4 waves x 8 rows x
+// 64 keys = 2048 keys; a workgroup owns a few consecutive tiles, so the
+// digit-major histogram has one column per workgroup (fewer scattered
+// histogram writes and a shorter histogram scan per pass)
 // ---------------------------------------------------------------------------
 constexpr int kMaxDigitBits = 10;
 constexpr int kMaxRadix = 1 << kMaxDigitBits;
 constexpr int kRows = 8;
 constexpr size_t kSortTile = static_cast<size_t>(kBlock) * kRows;
-constexpr int kTilesPerBlock = 4;
-constexpr size_t kSortSpan = kSortTile * kTilesPerBlock;
+// The scatter's tile is 8 waves x 4 or 8 rows (sort_plan).
+constexpr int kMaxTiles = 2;
+constexpr int kScatterWaves = 8;
+constexpr int kScatterBlock = kScatterWaves * 64;
+constexpr int kRowsSmall = 4;
+constexpr int kRowsLarge = 8;
 
 __device__ __forceinline__ uint64_t lanes_below(int lane) {
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -275,12 +279,12 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid, int db) 
 }
 
 // Per-workgroup digit counts of keys[...] >> bit (db-bit digits, the digit
-// masked to dmask), digit-major into hist, and the digit totals.  Dynamic
+// masked to dmask), digit-major into hist.  Dynamic
 // LDS: kWaves << db counters.
 template <typename K>
 __global__ __launch_bounds__(kBlock) void radix_upsweep_kernel(const K* __restrict__ keys,
                                                                size_t n, int bit, int db,
-                                                               uint32_t dmask,
+                                                               uint32_t dmask, int tiles,
                                                                uint32_t* __restrict__ hist,
                                                                size_t nb) {
     extern __shared__ uint32_t s_cnt[];  // [kWaves][R]
@@ -288,8 +292,8 @@ __global__ __launch_bounds__(kBlock) void radix_upsweep_kernel(const K* __restri
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < kWaves * R; i += kBlock) s_cnt[i] = 0;
     __syncthreads();
-    for (int t = 0; t < kTilesPerBlock; ++t) {
-        const size_t wave_base = blockIdx.x * kSortSpan + t * kSortTile +
+    for (int t = 0; t < tiles; ++t) {
+        const size_t wave_base = (static_cast<size_t>(blockIdx.x) * tiles + t) * kSortTile +
                                  static_cast<size_t>(wave) * kRows * 64;
         if (wave_base >= n) break;  // uniform over the wave
         K key[kRows];
@@ -326,32 +330,15 @@ __global__ __launch_bounds__(kBlock) void radix_upsweep_kernel(const K* __restri
     }
 }
 
-// One workgroup per digit d: the digit's total over the workgroups' counts
-// (its contiguous histogram row).
-__global__ __launch_bounds__(kBlock) void radix_digit_totals_kernel(const uint32_t* __restrict__ hist,
-                                                                    size_t nb,
-                                                                    uint32_t* __restrict__ digit_tot) {
-    __shared__ uint32_t s_wave[kWaves];
-    const uint32_t* row = hist + static_cast<size_t>(blockIdx.x) * nb;
-    uint32_t acc = 0;
-    for (size_t i = threadIdx.x; i < nb; i += kBlock) acc += row[i];
-    const uint32_t tot = block_sum<uint32_t, OpSum>(acc, s_wave);
-    if (threadIdx.x == 0) digit_tot[blockIdx.x] = tot;
-}
-
 // One workgroup per digit d: the exclusive scan of the workgroups' counts of
-// digit d (hist[d * nb + b], in place), offset by the number of keys with a
-// smaller digit -- the scatter positions of every (workgroup, digit).
+// digit d (hist[d * nb + b], in place), and the digit's total (the scatter adds
+// the start of every digit, an exclusive scan of the totals).
 __global__ __launch_bounds__(kBlock) void radix_offsets_kernel(uint32_t* __restrict__ hist,
                                                                size_t nb,
-                                                               const uint32_t* __restrict__ digit_tot) {
+                                                               uint32_t* __restrict__ digit_tot) {
     __shared__ uint32_t s_wave[kWaves];
-    const int d = blockIdx.x;
-    uint32_t below = 0;
-    for (int i = threadIdx.x; i < d; i += kBlock) below += digit_tot[i];
-    uint32_t carry = block_sum<uint32_t, OpSum>(below, s_wave);
-    __syncthreads();
-    uint32_t* row = hist + static_cast<size_t>(d) * nb;
+    uint32_t carry = 0;
+    uint32_t* row = hist + static_cast<size_t>(blockIdx.x) * nb;
     for (size_t chunk = 0; chunk < nb; chunk += kScanTile) {
         const size_t base = chunk + static_cast<size_t>(threadIdx.x) * kScanItems;
         uint32_t v[kScanItems];
@@ -373,64 +360,168 @@ __global__ __launch_bounds__(kBlock) void radix_offsets_kernel(uint32_t* __restr
         carry += tot;
         __syncthreads();
     }
+    if (threadIdx.x == 0) digit_tot[blockIdx.x] = carry;
 }
 
-// Stable scatter of one digit pass.  A tile's keys are first placed in LDS in
-// their sorted order within the tile (digit, then wave, then rank), then
-// written out by consecutive threads: the keys of one digit leave as one
-// contiguous run instead of one scattered store per key.  Dynamic LDS
-// (radix_scatter_lds): kWaves << db counters, 1 << db running positions,
-// 1 << db output bases, then the tile's staged keys and values.
-// Store: the last pass of an edge-store sort writes the store (st) instead of
-// keys_out / vals_out.
-template <typename K, typename V, bool Store = false>
-__global__ __launch_bounds__(kBlock) void radix_scatter_kernel(
-    const K* __restrict__ keys_in, const V* __restrict__ vals_in, K* __restrict__ keys_out,
-    V* __restrict__ vals_out, size_t n, int bit, int db, uint32_t dmask,
-    const uint32_t* __restrict__ offsets, size_t nb, SortedStore st = SortedStore{}) {
-    extern __shared__ __align__(16) uint32_t s_lds[];
-    __shared__ uint32_t s_wave[kWaves];
-    const int R = 1 << db;
-    uint32_t* s_cnt = s_lds;                // [kWaves][R]: counts, then tile-local offsets
-    uint32_t* s_run = s_cnt + kWaves * R;   // the workgroup's next output position per digit
-    uint32_t* s_base = s_run + R;           // output position of tile-local position 0, per digit
-    K* s_key = reinterpret_cast<K*>(s_base + R);
-    V* s_val = reinterpret_cast<V*>(s_key + kSortTile);
+// The digit pass's LDS for a tile of W waves x Rows rows: W * R counters, R
+// running positions, R output bases, then the tile's staged keys and values.
+template <int W, int Rows, typename K, typename V>
+struct TileLds {
+    static constexpr size_t kTile = static_cast<size_t>(W) * Rows * 64;
+    uint32_t* cnt;   // [W][R]: counts, then tile-local offsets
+    uint32_t* run;   // the workgroup's next output position per digit
+    uint32_t* base;  // output position of tile-local position 0, per digit
+    K* key;
+    V* val;
+    __device__ __forceinline__ TileLds(uint32_t* lds, int R) {
+        cnt = lds;
+        run = cnt + W * R;
+        base = run + R;
+        key = reinterpret_cast<K*>(base + R);
+        val = reinterpret_cast<V*>(key + kTile);
+    }
+    static size_t bytes(int R) {
+        return (static_cast<size_t>(W) + 2) * R * sizeof(uint32_t) + kTile * (sizeof(K) + sizeof(V));
+    }
+};
+
+// One tile's keys, values, digits and ranks in registers: row r of wave w is
+// keys [(w * Rows + r) * 64, + 64) of the tile.
+template <int Rows, typename K, typename V>
+struct TileRegs {
+    K key[Rows];
+    V val[Rows];
+    uint32_t dig[Rows];
+    uint32_t rank[Rows];
+};
+
+template <int W, int Rows, typename K, typename V>
+__device__ __forceinline__ void tile_load(const K* __restrict__ keys_in,
+                                          const V* __restrict__ vals_in, size_t n, size_t tile_base,
+                                          TileRegs<Rows, K, V>& t) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t wave_base = tile_base + static_cast<size_t>(wave) * Rows * 64;
+#pragma unroll
+    for (int r = 0; r < Rows; ++r) {
+        const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
+        const bool valid = i < n;
+        t.key[r] = valid ? keys_in[i] : K(0);
+        t.val[r] = (valid && vals_in) ? vals_in[i] : V(0);
+    }
+}
+
+// Ranks the loaded tile's keys by digit: rank = the number of earlier keys of
+// the wave with the same digit; l.cnt[wave][d] ends as the wave's count of
+// digit d.  The counters must be zero.
+template <int W, int Rows, typename K, typename V>
+__device__ __forceinline__ void tile_rank(size_t n, size_t tile_base, int bit, int db,
+                                          uint32_t dmask, const TileLds<W, Rows, K, V>& l,
+                                          TileRegs<Rows, K, V>& t) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, R = 1 << db;
+    const size_t wave_base = tile_base + static_cast<size_t>(wave) * Rows * 64;
+#pragma unroll
+    for (int r = 0; r < Rows; ++r) {
+        const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
+        const bool valid = i < n;
+        const uint32_t d = static_cast<uint32_t>(t.key[r] >> bit) & dmask;
+        t.dig[r] = d;
+        const uint64_t m = match_digit(d, valid, db);
+        const uint32_t before = __popcll(m & lanes_below(lane));
+        const uint32_t prior = l.cnt[wave * R + d];
+        t.rank[r] = prior + before;
+        if (valid && before == 0) l.cnt[wave * R + d] = prior + __popcll(m);
+    }
+}
+
+// Stages the ranked tile in LDS in its sorted order, l.cnt holding the
+// tile-local start of every (wave, digit).
+template <int W, int Rows, typename K, typename V>
+__device__ __forceinline__ void tile_stage(size_t n, size_t tile_base, int db, bool with_vals,
+                                           const TileLds<W, Rows, K, V>& l,
+                                           const TileRegs<Rows, K, V>& t) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, R = 1 << db;
+    const size_t wave_base = tile_base + static_cast<size_t>(wave) * Rows * 64;
+#pragma unroll
+    for (int r = 0; r < Rows; ++r) {
+        const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
+        if (i < n) {
+            const uint32_t lp = l.cnt[wave * R + t.dig[r]] + t.rank[r];
+            l.key[lp] = t.key[r];
+            if (with_vals) l.val[lp] = t.val[r];
+        }
+    }
+}
+
+// Writes the staged tile out by consecutive threads, so each digit's keys
+// leave as one contiguous run: key lp goes to l.base[digit] + lp.  Store: the
+// store (st) is written instead of keys_out / vals_out.
+template <bool Store, int W, int Rows, typename K, typename V>
+__device__ __forceinline__ void tile_write(size_t n, size_t tile_base, int bit, uint32_t dmask,
+                                           const TileLds<W, Rows, K, V>& l, K* __restrict__ keys_out,
+                                           V* __restrict__ vals_out, const SortedStore& st) {
+    constexpr size_t kTile = TileLds<W, Rows, K, V>::kTile;
+    const size_t tile_n = n - tile_base < kTile ? n - tile_base : kTile;
+#pragma unroll
+    for (int r = 0; r < Rows; ++r) {
+        const uint32_t lp = static_cast<uint32_t>(r) * W * 64 + threadIdx.x;
+        if (lp < tile_n) {
+            const K k = l.key[lp];
+            const uint32_t d = static_cast<uint32_t>(k >> bit) & dmask;
+            const uint32_t pos = l.base[d] + lp;
+            if constexpr (Store) {
+                const uint64_t v = l.val[lp];
+                st.src[pos] = static_cast<int32_t>(static_cast<uint32_t>(v));
+                st.dst[pos] = static_cast<int32_t>(static_cast<uint32_t>(v >> 32));
+                st.ts[pos] = static_cast<int64_t>(static_cast<uint64_t>(k) +
+                                                  static_cast<uint64_t>(st.tmin));
+            } else {
+                keys_out[pos] = k;
+                if (vals_out) vals_out[pos] = l.val[lp];
+            }
+        }
+    }
+}
+
+// Stable scatter of one digit pass, `tiles` tiles per workgroup.  Dynamic LDS:
+// TileLds::bytes.
+template <typename K, typename V, int Rows, bool Store = false>
+__global__ __launch_bounds__(kScatterBlock) void radix_scatter_kernel(
+    const K* __restrict__ keys_in, const V* __restrict__ vals_in, K* __restrict__ keys_out,
+    V* __restrict__ vals_out, size_t n, int bit, int db, uint32_t dmask, int tiles,
+    const uint32_t* __restrict__ offsets, size_t nb, const uint32_t* __restrict__ digit_tot,
+    SortedStore st = SortedStore{}) {
+    extern __shared__ __align__(16) uint32_t s_lds[];
+    __shared__ uint32_t s_wave[kScatterWaves];
+    const int R = 1 << db;
+    constexpr size_t kTile = static_cast<size_t>(kScatterBlock) * Rows;
+    const TileLds<kScatterWaves, Rows, K, V> l(s_lds, R);
     // digits [d0, d0 + per) of this thread in the tile epilogue
-    const int per = (R + kBlock - 1) / kBlock;
+    const int per = (R + kScatterBlock - 1) / kScatterBlock;
     const int d0 = threadIdx.x * per;
-    for (int d = threadIdx.x; d < R; d += kBlock)
-        s_run[d] = offsets[static_cast<size_t>(d) * nb + blockIdx.x];
-    for (int t = 0; t < kTilesPerBlock; ++t) {
-        const size_t tile_base = blockIdx.x * kSortSpan + t * kSortTile;
+    {
+        // the workgroup's first output position of every digit: the keys of
+        // smaller digits, then those of earlier workgroups
+        uint32_t mine = 0;
+        for (int j = 0; j < per; ++j)
+            if (d0 + j < R) mine += digit_tot[d0 + j];
+        uint32_t tot;
+        uint32_t at = block_exclusive_scan<uint32_t, OpSum, kScatterWaves>(mine, &tot, s_wave);
+        for (int j = 0; j < per; ++j) {
+            const int d = d0 + j;
+            if (d < R) {
+                l.run[d] = at + offsets[static_cast<size_t>(d) * nb + blockIdx.x];
+                at += digit_tot[d];
+            }
+        }
+    }
+    for (int t = 0; t < tiles; ++t) {
+        const size_t tile_base = (static_cast<size_t>(blockIdx.x) * tiles + t) * kTile;
         if (tile_base >= n) break;  // uniform over the workgroup
-        for (int i = threadIdx.x; i < kWaves * R; i += kBlock) s_cnt[i] = 0;
+        for (int i = threadIdx.x; i < kScatterWaves * R; i += kScatterBlock) l.cnt[i] = 0;
         __syncthreads();
-        const size_t wave_base = tile_base + static_cast<size_t>(wave) * kRows * 64;
-        K key[kRows];
-        V val[kRows];
-        uint32_t dig[kRows];
-        uint32_t rank[kRows];
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
-            const bool valid = i < n;
-            key[r] = valid ? keys_in[i] : K(0);
-            val[r] = (valid && vals_in) ? vals_in[i] : V(0);
-        }
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
-            const bool valid = i < n;
-            const uint32_t d = static_cast<uint32_t>(key[r] >> bit) & dmask;
-            dig[r] = d;
-            const uint64_t m = match_digit(d, valid, db);
-            const uint32_t before = __popcll(m & lanes_below(lane));
-            const uint32_t prior = s_cnt[wave * R + d];
-            rank[r] = prior + before;
-            if (valid && before == 0) s_cnt[wave * R + d] = prior + __popcll(m);
-        }
+        TileRegs<Rows, K, V> regs;
+        tile_load<kScatterWaves>(keys_in, vals_in, n, tile_base, regs);
+        tile_rank(n, tile_base, bit, db, dmask, l, regs);
         __syncthreads();
         {
             // tile epilogue: the tile-local start of every digit (an exclusive
@@ -441,115 +532,209 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(
                 const int d = d0 + j;
                 if (d < R) {
 #pragma unroll
-                    for (int w = 0; w < kWaves; ++w) cnt_mine += s_cnt[w * R + d];
+                    for (int w = 0; w < kScatterWaves; ++w) cnt_mine += l.cnt[w * R + d];
                 }
             }
             uint32_t tot;
-            uint32_t start = block_exclusive_scan<uint32_t, OpSum>(cnt_mine, &tot, s_wave);
+            uint32_t start = block_exclusive_scan<uint32_t, OpSum, kScatterWaves>(cnt_mine, &tot, s_wave);
             for (int j = 0; j < per; ++j) {
                 const int d = d0 + j;
                 if (d < R) {
                     const uint32_t first = start;
 #pragma unroll
-                    for (int w = 0; w < kWaves; ++w) {
-                        const uint32_t c = s_cnt[w * R + d];
-                        s_cnt[w * R + d] = start;
+                    for (int w = 0; w < kScatterWaves; ++w) {
+                        const uint32_t c = l.cnt[w * R + d];
+                        l.cnt[w * R + d] = start;
                         start += c;
                     }
-                    s_base[d] = s_run[d] - first;  // wraps back in pos = base + local
-                    s_run[d] += start - first;
+                    l.base[d] = l.run[d] - first;  // wraps back in pos = base + local
+                    l.run[d] += start - first;
                 }
             }
         }
         __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
-            if (i < n) {
-                const uint32_t lp = s_cnt[wave * R + dig[r]] + rank[r];
-                s_key[lp] = key[r];
-                if (vals_out || Store) s_val[lp] = val[r];  // the store pass writes no vals_out
-            }
-        }
+        // the store pass writes no vals_out
+        tile_stage(n, tile_base, db, vals_out || Store, l, regs);
         __syncthreads();
-        const size_t tile_n = n - tile_base < kSortTile ? n - tile_base : kSortTile;
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            const uint32_t lp = static_cast<uint32_t>(r) * kBlock + threadIdx.x;
-            if (lp < tile_n) {
-                const K k = s_key[lp];
-                const uint32_t d = static_cast<uint32_t>(k >> bit) & dmask;
-                const uint32_t pos = s_base[d] + lp;
-                if constexpr (Store) {
-                    const uint64_t v = s_val[lp];
-                    st.src[pos] = static_cast<int32_t>(static_cast<uint32_t>(v));
-                    st.dst[pos] = static_cast<int32_t>(static_cast<uint32_t>(v >> 32));
-                    st.ts[pos] = static_cast<int64_t>(static_cast<uint64_t>(k) +
-                                                      static_cast<uint64_t>(st.tmin));
-                } else {
-                    keys_out[pos] = k;
-                    if (vals_out) vals_out[pos] = s_val[lp];
-                }
-            }
-        }
-        __syncthreads();  // s_cnt and the staging are reused by the next tile
+        tile_write<Store>(n, tile_base, bit, dmask, l, keys_out, vals_out, st);
+        __syncthreads();  // the counters and the staging are reused by the next tile
     }
 }
 
-template <typename K, typename V>
-size_t radix_scatter_lds(int R) {
-    return (static_cast<size_t>(kWaves) + 2) * R * sizeof(uint32_t) +
-           kSortTile * (sizeof(K) + sizeof(V));
+// ---------------------------------------------------------------------------
+// sorts of one tile: every digit pass in one workgroup
+// ---------------------------------------------------------------------------
+// A sort this small is latency only (launches, and each pass's chain of LDS
+// phases), so the tile is spread over 16 waves of 2 rows and a digit has at
+// most 8 bits (a digit per thread between the passes).  320 keys by 32 bits:
+// 14 us against 51 us as three kernels per pass.
+constexpr int kTileBlock = 1024;
+constexpr int kTileWaves = kTileBlock / 64;
+constexpr int kTileRows = 2;
+constexpr size_t kTileKeys = static_cast<size_t>(kTileBlock) * kTileRows;
+constexpr int kTileDigitBits = 8;
+
+// The keys go round through LDS.  keys_out / vals_out may be the inputs.
+template <typename K, typename V, bool Store = false>
+__global__ __launch_bounds__(kTileBlock) void radix_tile_sort_kernel(
+    const K* keys_in, const V* vals_in, K* keys_out, V* vals_out, uint32_t n, int begin_bit,
+    int end_bit, int db, SortedStore st = SortedStore{}) {
+    extern __shared__ __align__(16) uint32_t s_lds[];
+    __shared__ uint32_t s_wave[kTileWaves];
+    const int R = 1 << db;
+    const TileLds<kTileWaves, kTileRows, K, V> l(s_lds, R);
+    TileRegs<kTileRows, K, V> regs;
+    tile_load<kTileWaves>(keys_in, vals_in, n, 0, regs);
+    for (int i = threadIdx.x; i < R; i += kTileBlock) l.base[i] = 0;
+    const int d = threadIdx.x;
+    for (int bit = begin_bit; bit < end_bit; bit += db) {
+        const int w = end_bit - bit < db ? end_bit - bit : db;
+        const uint32_t dmask = (1u << w) - 1u;
+        if (bit != begin_bit) {
+            // the keys as the last pass left them (every wave's reads precede
+            // the next staging: the barriers below)
+            tile_load<kTileWaves>(static_cast<const K*>(l.key),
+                                   vals_in ? static_cast<const V*>(l.val) : nullptr, n, 0, regs);
+        }
+        for (int i = threadIdx.x; i < kTileWaves * R; i += kTileBlock) l.cnt[i] = 0;
+        __syncthreads();
+        tile_rank(n, 0, bit, db, dmask, l, regs);
+        __syncthreads();
+        uint32_t c = 0;
+        if (d < R) {
+#pragma unroll
+            for (int q = 0; q < kTileWaves; ++q) c += l.cnt[q * R + d];
+        }
+        uint32_t tot;
+        uint32_t start = block_exclusive_scan<uint32_t, OpSum, kTileWaves>(c, &tot, s_wave);
+        if (d < R) {
+#pragma unroll
+            for (int q = 0; q < kTileWaves; ++q) {
+                const uint32_t x = l.cnt[q * R + d];
+                l.cnt[q * R + d] = start;
+                start += x;
+            }
+        }
+        __syncthreads();
+        tile_stage(n, 0, db, vals_in != nullptr, l, regs);
+        __syncthreads();
+    }
+    tile_write<Store>(n, 0, 0, 0u, l, keys_out, vals_out, st);  // base[0] = 0: key lp to lp
 }
 
-// hist layout: nb * kMaxRadix per-workgroup counts, then kMaxPasses *
-// kMaxRadix digit totals (one row per pass, cleared once per sort).
-constexpr int kMaxPasses = (64 + kMaxDigitBits - 1) / kMaxDigitBits;
+// How a sort of n keys by `bits` bits runs with `words` words of scratch: in
+// one workgroup when they fit its tile, else three kernels per pass.  Measured
+// (us; keys with 64-bit values, uniform):
+//  - Digits: up to 10 bits while launches are the cost (100k keys by 20 bits:
+//    43 in two passes, 47 in three), up to 8 past kWideMax, where a wide
+//    digit's short runs write partial lines (1M: 81 in two passes of 10 bits,
+//    60 in three of 7; 20M: 772 and 542).
+//  - Tiles: one per workgroup until kSortBlocks workgroups (a workgroup's
+//    tiles run one after the other: 100k keys by 32 bits, 64 with one, 90 with
+//    two, 145 with four), then two.
+//  - Rows: 2048-key tiles keep more workgroups resident (9M keys by 20 bits:
+//    216 against 230); from kLargeMin keys on the output no longer stays in
+//    cache, and 4096-key tiles write longer runs (20M: 480 against 528; 50M by
+//    27 bits: 1716 against 1996).
+constexpr size_t kWideMax = size_t{1} << 19;
+constexpr size_t kLargeMin = size_t{3} << 22;
+constexpr int kDigitBits = 8;
+constexpr size_t kSortBlocks = 1024;
 
-// Passes and digit width of a sort of `bits` key bits.
-int sort_passes(int bits) { return (bits + kMaxDigitBits - 1) / kMaxDigitBits; }
-int sort_digit_bits(int bits) {
-    const int p = sort_passes(bits);
-    return (bits + p - 1) / p;
+struct SortPlan {
+    bool one_tile, large;
+    int passes, db;
+    int tiles;     // tiles per workgroup
+    size_t nb;     // workgroups of a pass
+    size_t words;  // scratch: per-workgroup counts, then the digit totals
+};
+
+SortPlan sort_plan(size_t n, int bits, size_t words) {
+    SortPlan p{};
+    p.one_tile = n <= kTileKeys;
+    p.large = n >= kLargeMin;
+    const int most = p.one_tile ? kTileDigitBits : n <= kWideMax ? kMaxDigitBits : kDigitBits;
+    p.passes = (bits + most - 1) / most;
+    p.db = (bits + p.passes - 1) / p.passes;
+    if (p.one_tile) return p;
+    const size_t tile = static_cast<size_t>(kScatterBlock) * (p.large ? kRowsLarge : kRowsSmall);
+    const size_t R = size_t{1} << p.db, all = (n + tile - 1) / tile;
+    for (p.tiles = 1;; p.tiles *= 2) {
+        p.nb = (all + p.tiles - 1) / p.tiles;
+        p.words = p.nb * R + R;
+        if (p.tiles >= kMaxTiles || (p.nb <= kSortBlocks && p.words <= words)) return p;
+    }
+}
+
+// One digit pass's scatter (st: the store to write instead, or nullptr).
+template <int Rows, typename K, typename V>
+void launch_scatter(const SortPlan& p, const K* ki, const V* vi, K* ko, V* vo, size_t n, int bit,
+                    uint32_t dmask, const uint32_t* offsets, const uint32_t* totals,
+                    const SortedStore* st, hipStream_t s) {
+    const size_t lds = TileLds<kScatterWaves, Rows, K, V>::bytes(1 << p.db);
+    if constexpr (std::is_same<V, uint64_t>::value) {
+        if (st) {
+            hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows, true>), dim3(p.nb),
+                               dim3(kScatterBlock), lds, s, ki, vi, nullptr, nullptr, n, bit, p.db,
+                               dmask, p.tiles, offsets, p.nb, totals, *st);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows>), dim3(p.nb), dim3(kScatterBlock), lds, s,
+                       ki, vi, ko, vo, n, bit, p.db, dmask, p.tiles, offsets, p.nb, totals);
 }
 
 template <typename K, typename V = uint32_t>
 int radix_sort_impl(K* keys0, V* vals0, K* keys1, V* vals1, size_t n,
-                    int begin_bit, int end_bit, uint32_t* hist, hipStream_t s,
+                    int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
                     const SortedStore* store = nullptr) {
     if (n <= 1 || end_bit <= begin_bit) return 0;
-    const size_t nb = (n + kSortSpan - 1) / kSortSpan;
-    const int passes = sort_passes(end_bit - begin_bit);
-    const int db = sort_digit_bits(end_bit - begin_bit);
-    const int R = 1 << db;
-    uint32_t* totals = hist + nb * kMaxRadix;
-    const size_t lds_up = static_cast<size_t>(kWaves) * R * sizeof(uint32_t);
-    const size_t lds_sc = radix_scatter_lds<K, V>(R);
-    int cur = 0;
+    const SortPlan p = sort_plan(n, end_bit - begin_bit, tmp.n);
+    if (p.words > tmp.n) throw std::runtime_error("radix sort: scratch too small");
+    const int db = p.db;
+    const size_t R = size_t{1} << db, nb = p.nb;
     K* kb[2] = {keys0, keys1};
     V* vb[2] = {vals0, vals1};
-    for (int pass = 0; pass < passes; ++pass) {
+    constexpr bool can_store = std::is_same<V, uint64_t>::value;
+    if (p.one_tile) {
+        const size_t lds = TileLds<kTileWaves, kTileRows, K, V>::bytes(static_cast<int>(R));
+        const int out = p.passes & 1;
+        bool stored = false;
+        if constexpr (can_store) {
+            if (store) {
+                hipLaunchKernelGGL((radix_tile_sort_kernel<K, V, true>), dim3(1), dim3(kTileBlock),
+                                   lds, s, kb[0], vb[0], nullptr, nullptr,
+                                   static_cast<uint32_t>(n), begin_bit, end_bit, db, *store);
+                stored = true;
+            }
+        }
+        if (!stored)
+            hipLaunchKernelGGL((radix_tile_sort_kernel<K, V>), dim3(1), dim3(kTileBlock), lds, s,
+                               kb[0], vb[0], kb[out], vb[out], static_cast<uint32_t>(n), begin_bit,
+                               end_bit, db);
+        check_hip(hipGetLastError(), "radix sort launch");
+        return out;
+    }
+    uint32_t* totals = tmp.p + nb * R;
+    const size_t tile = static_cast<size_t>(kScatterBlock) * (p.large ? kRowsLarge : kRowsSmall);
+    const int up_tiles = static_cast<int>(p.tiles * tile / kSortTile);
+    int cur = 0;
+    for (int pass = 0; pass < p.passes; ++pass) {
         const int bit = begin_bit + pass * db;
         // the last digit stops at end_bit
         const int w = end_bit - bit < db ? end_bit - bit : db;
         const uint32_t dmask = (1u << w) - 1u;
-        uint32_t* tot = totals + pass * R;
-        hipLaunchKernelGGL((radix_upsweep_kernel<K>), dim3(nb), dim3(kBlock), lds_up, s, kb[cur],
-                           n, bit, db, dmask, hist, nb);
-        hipLaunchKernelGGL(radix_digit_totals_kernel, dim3(R), dim3(kBlock), 0, s, hist, nb, tot);
-        hipLaunchKernelGGL(radix_offsets_kernel, dim3(R), dim3(kBlock), 0, s, hist, nb, tot);
-        if constexpr (std::is_same<V, uint64_t>::value) {
-            if (store && pass == passes - 1) {
-                hipLaunchKernelGGL((radix_scatter_kernel<K, V, true>), dim3(nb), dim3(kBlock),
-                                   lds_sc, s, kb[cur], vb[cur], nullptr, nullptr, n, bit, db,
-                                   dmask, hist, nb, *store);
-                check_hip(hipGetLastError(), "radix sort launch");
-                return cur ^ 1;
-            }
-        }
-        hipLaunchKernelGGL((radix_scatter_kernel<K, V>), dim3(nb), dim3(kBlock), lds_sc, s,
-                           kb[cur], vb[cur], kb[cur ^ 1], vb[cur ^ 1], n, bit, db, dmask, hist,
-                           nb);
+        hipLaunchKernelGGL((radix_upsweep_kernel<K>), dim3(nb), dim3(kBlock),
+                           kWaves * R * sizeof(uint32_t), s, kb[cur], n, bit, db, dmask, up_tiles,
+                           tmp.p, nb);
+        hipLaunchKernelGGL(radix_offsets_kernel, dim3(R), dim3(kBlock), 0, s, tmp.p, nb, totals);
+        const SortedStore* st = pass == p.passes - 1 ? store : nullptr;
+        if (p.large)
+            launch_scatter<kRowsLarge>(p, kb[cur], vb[cur], kb[cur ^ 1], vb[cur ^ 1], n, bit, dmask,
+                                       tmp.p, totals, st, s);
+        else
+            launch_scatter<kRowsSmall>(p, kb[cur], vb[cur], kb[cur ^ 1], vb[cur ^ 1], n, bit, dmask,
+                                       tmp.p, totals, st, s);
         check_hip(hipGetLastError(), "radix sort launch");
         cur ^= 1;
     }
@@ -681,8 +866,11 @@ int reduce_blocks(size_t n) {
 }  // namespace
 
 size_t scan_scratch_elems(size_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
-size_t radix_hist_elems(size_t n) {
-    return ((n + kSortSpan - 1) / kSortSpan) * kMaxRadix + kMaxPasses * kMaxRadix;
+size_t radix_tmp_elems(size_t n, int bits) {
+    return n <= 1 || bits <= 0 ? 1 : std::max<size_t>(sort_plan(n, bits, SIZE_MAX).words, 1);
+}
+size_t radix_min_elems(size_t n, int bits) {
+    return n <= 1 || bits <= 0 ? 1 : std::max<size_t>(sort_plan(n, bits, 0).words, 1);
 }
 
 void exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* scratch,
@@ -711,39 +899,39 @@ void running_max_f64(double* data, size_t n, double* scratch, hipStream_t s) {
 }
 
 int radix_sort_u64(uint64_t* keys0, uint32_t* vals0, uint64_t* keys1, uint32_t* vals1, size_t n,
-                   int begin_bit, int end_bit, uint32_t* hist, hipStream_t s) {
-    return radix_sort_impl<uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, hist, s);
+                   int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
+    return radix_sort_impl<uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s);
 }
 int radix_sort_u32(uint32_t* keys0, uint32_t* vals0, uint32_t* keys1, uint32_t* vals1, size_t n,
-                   int begin_bit, int end_bit, uint32_t* hist, hipStream_t s) {
-    return radix_sort_impl<uint32_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, hist, s);
+                   int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
+    return radix_sort_impl<uint32_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s);
 }
 int radix_sort_u64_v64(uint64_t* keys0, uint64_t* vals0, uint64_t* keys1, uint64_t* vals1,
-                       size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s) {
+                       size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
     return radix_sort_impl<uint64_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit,
-                                               hist, s);
+                                               tmp, s);
 }
 int radix_sort_u32_v64(uint32_t* keys0, uint64_t* vals0, uint32_t* keys1, uint64_t* vals1,
-                       size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s) {
+                       size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
     return radix_sort_impl<uint32_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit,
-                                               hist, s);
+                                               tmp, s);
 }
-int radix_passes(int begin_bit, int end_bit) {
-    return end_bit > begin_bit ? sort_passes(end_bit - begin_bit) : 0;
+int radix_passes(size_t n, int begin_bit, int end_bit) {
+    return n > 1 && end_bit > begin_bit ? sort_plan(n, end_bit - begin_bit, SIZE_MAX).passes : 0;
 }
 bool radix_sort_u32_v64_store(uint32_t* keys0, uint64_t* vals0, uint32_t* keys1, uint64_t* vals1,
-                              size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s,
+                              size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
                               const SortedStore& out) {
     if (n <= 1 || end_bit <= begin_bit) return false;
-    radix_sort_impl<uint32_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, hist, s,
+    radix_sort_impl<uint32_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s,
                                         &out);
     return true;
 }
 bool radix_sort_u64_v64_store(uint64_t* keys0, uint64_t* vals0, uint64_t* keys1, uint64_t* vals1,
-                              size_t n, int begin_bit, int end_bit, uint32_t* hist, hipStream_t s,
+                              size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
                               const SortedStore& out) {
     if (n <= 1 || end_bit <= begin_bit) return false;
-    radix_sort_impl<uint64_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, hist, s,
+    radix_sort_impl<uint64_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s,
                                         &out);
     return true;
 }

@@ -1859,7 +1859,7 @@ __global__ __launch_bounds__(kB) void walk_stats_kernel(const int32_t* __restric
 // per device (with that device current) when the first handle on it is
 // created, and only that address is handed to kernels and copies.  Calls on
 // one device share the array, so overlapping calls race.
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes + kNoAllocSortBytes];
 
 namespace {
 std::mutex g_scratch_mu;
@@ -1971,7 +1971,7 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
                 const size_t m = cfg.is_directed ? last_n : 2 * last_n;
                 uint32_t* ka = sp.take(k32a, m);
                 uint32_t* kb = sp.take(k32b, m);
-                uint32_t* hi = sp.take(hist, radix_hist_elems(m));
+                const RadixTmp hi = sp.sort_tmp(hist, m, 32);
                 uint32_t* fl = sp.take(flags, m + 1);
                 uint32_t* sc = sp.take(scan, m + 1);
                 uint32_t* ss = sp.take(scan_scratch, scan_scratch_elems(m + 1));
@@ -2060,7 +2060,7 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
         uint32_t* kb = sp.take(k32b, nw);
         uint32_t* va = sp.take(v32a, nw);
         uint32_t* vb = sp.take(v32b, nw);
-        uint32_t* hi = sp.take(hist, radix_hist_elems(nw));
+        const RadixTmp hi = sp.sort_tmp(hist, nw, 32);
         hipLaunchKernelGGL(random_keys_kernel, dim3(grid_for(nw)), dim3(kB), 0, s, nw,
                            static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32), ka, va);
         const int w = radix_sort_u32(ka, va, kb, vb, nw, 0, 32, hi, s);
@@ -2305,8 +2305,8 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
         if (sorted) {
             uint32_t* kb = sp.take(k32b, nw);
             uint32_t* vb = sp.take(v32b, nw);
-            uint32_t* hi = sp.take(hist, radix_hist_elems(nw));
             const int bits = std::max(1, 32 - __builtin_clz(none | 1u));
+            const RadixTmp hi = sp.sort_tmp(hist, nw, bits);
             const int wsort = radix_sort_u32(ka, va, kb, vb, nw, 0, bits, hi, s);
             a.order = wsort ? vb : va;
             a.xcd_remap = 1;
@@ -2335,9 +2335,9 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
         WalkCarry* carry = reinterpret_cast<WalkCarry*>(sp.take(ng_carry, 8 * nw));
         uint32_t* kb[2] = {sp.take(ng_keys0, nw), sp.take(ng_keys1, nw)};
         uint32_t* vb[2] = {sp.take(ng_vals0, nw), sp.take(ng_vals1, nw)};
-        uint32_t* hi = sp.take(hist, radix_hist_elems(nw));
-        uint32_t* cnt = sp.take(ng_count, 1);
         const int nbits = std::max(1, bit_length(static_cast<uint64_t>(std::max(max_node_id, 0))));
+        const RadixTmp hi = sp.sort_tmp(hist, nw, nbits);
+        uint32_t* cnt = sp.take(ng_count, 1);
         check_hip(hipMemsetAsync(cnt, 0, 4, s), "live count clear");
         int in = 0;  // the pair the next list is emitted into
         TRW_LAUNCH(node_group_init_kernel, dim3(grid_for(nw)), g, a, carry, kb[in], vb[in], cnt);

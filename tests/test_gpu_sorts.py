@@ -1,0 +1,43 @@
+"""The build's radix sorts at the edges of their forms (one tile in one
+workgroup, wide and narrow digits, one and two tiles per workgroup, the large
+tile), through the arrays they order: the edge store is stable by timestamp
+and the node index stable by (node, position), which numpy's stable argsort
+gives exactly."""
+import numpy as np
+import pytest
+
+from temporal_random_walk import capi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("directed", [True, False])
+@pytest.mark.parametrize("n,ts_bits", [
+    (1, 8), (2, 1), (64, 33), (1023, 20), (2047, 8), (2048, 9), (2049, 9), (4097, 33),
+    (100_001, 20), (262_145, 27), (524_288, 20), (524_289, 20), (2_097_153, 30),
+    (6_291_456, 17), (12_582_912, 12),
+])
+def test_store_and_node_index_order_at_the_sort_forms_edges(n, ts_bits, directed):
+    if n > 6_291_456 and not directed:
+        pytest.skip("the undirected index of half as many edges sorts as many entries")
+    rng = np.random.default_rng(n + ts_bits)
+    nodes = max(2, n // 7)
+    src = rng.integers(0, nodes, n).astype(np.int32)
+    src[rng.random(n) < 0.4] = nodes // 2  # a hub: rows of one digit
+    dst = rng.integers(0, nodes, n).astype(np.int32)
+    ts = rng.integers(0, 1 << ts_bits, n).astype(np.int64) - 5
+    eng = capi.Engine(is_directed=directed)
+    eng.add_edges(src, dst, ts)
+    order = np.argsort(ts, kind="stable")
+    s, d = src[order], dst[order]
+    np.testing.assert_array_equal(eng.array("timestamps"), ts[order])
+    np.testing.assert_array_equal(eng.array("sources"), s)
+    np.testing.assert_array_equal(eng.array("targets"), d)
+    if directed:
+        out, inn = np.argsort(s, kind="stable"), np.argsort(d, kind="stable")
+        np.testing.assert_array_equal(eng.array("node_ts_sorted_inbound_indices"), inn)
+    else:  # entries 2i and 2i + 1 are edge i seen from its endpoints
+        both = np.stack([s, d], axis=1).ravel()
+        out = np.argsort(both, kind="stable") // 2
+    np.testing.assert_array_equal(eng.array("node_ts_sorted_outbound_indices"), out)
+    eng.close()
