@@ -347,8 +347,10 @@ typedef struct trw_walk_stats {
                                    * (no scratch, no layout pass); 0: scratch
                                    * and the layout pass */
     uint64_t slot_word_format;    /* what a walk slot's 64-bit word held: 0 node,
-                                   * timestamp rank and edge id; 1 node and edge
-                                   * id (the three do not fit in 64 bits) */
+                                   * time key (timestamp rank or offset) and edge
+                                   * id; 1 the three do not fit in 64 bits: node
+                                   * and edge id, with the key's offset in the
+                                   * edge's block where there is room for it */
 } trw_walk_stats;
 trw_status trw_get_walk_stats(void* handle, trw_walk_stats* out);
 

@@ -167,11 +167,13 @@ __global__ void ts_group_scatter_kernel(const int64_t* __restrict__ ts, size_t n
                                         const uint32_t* __restrict__ flags,
                                         const uint32_t* __restrict__ scan,
                                         uint32_t* __restrict__ off, int64_t* __restrict__ uq,
+                                        int time_keys, int64_t t0,
                                         uint32_t* __restrict__ erank) {
     const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
     if (i >= n) return;
+    // the time key: the offset from the store's first timestamp, or the
     // exclusive scan of the group-start flags: the group index of position i
-    erank[i] = scan[i] + flags[i] - 1u;
+    erank[i] = time_keys ? static_cast<uint32_t>(ts[i] - t0) : scan[i] + flags[i] - 1u;
     if (flags[i]) {
         off[scan[i]] = static_cast<uint32_t>(i);
         uq[scan[i]] = ts[i];
@@ -179,17 +181,48 @@ __global__ void ts_group_scatter_kernel(const int64_t* __restrict__ ts, size_t n
     if (i == n - 1) off[scan[n]] = static_cast<uint32_t>(n);
 }
 
-// Rank of timestamp -1 among the unique timestamps, or -2 when no edge has it:
-// the walk compares ranks with it for the reference's `ts == -1` tests.
-__global__ void neg1_rank_kernel(const int64_t* __restrict__ uq, uint32_t T,
-                                 int32_t* __restrict__ out) {
+// Key of timestamp -1, or -2 when no edge has it: the walk compares keys with
+// it for the reference's `ts == -1` tests.
+__global__ void neg1_rank_kernel(const int64_t* __restrict__ uq, uint32_t T, int time_keys,
+                                 int64_t t0, int32_t* __restrict__ out) {
     uint32_t lo = 0, hi = T;
     while (lo < hi) {
         const uint32_t mid = lo + ((hi - lo) >> 1);
         if (uq[mid] < -1) lo = mid + 1;
         else hi = mid;
     }
-    *out = (lo < T && uq[lo] == -1) ? static_cast<int32_t>(lo) : -2;
+    *out = (lo < T && uq[lo] == -1)
+               ? static_cast<int32_t>(time_keys ? -1 - t0 : static_cast<int64_t>(lo))
+               : -2;
+}
+
+// The key blocks of a slot word with `bits` bits for a key (index_layout.h):
+// the largest shift whose blocks of 2^shift edges each span less than
+// 2^bits - 1 keys, with at most kMaxKeyBlocks of them, into out[0] (or
+// kNoKeyBlocks), then the blocks' first keys.  One workgroup: each shift reads
+// two keys of at most kMaxKeyBlocks blocks.
+__global__ __launch_bounds__(1024) void key_block_table_kernel(const uint32_t* __restrict__ key,
+                                                               uint64_t n, int bits,
+                                                               uint32_t* __restrict__ out) {
+    const uint32_t limit = bits >= 32 ? 0xffffffffu : (1u << bits) - 2u;  // largest span
+    int found = -1;
+    for (int sh = 31; sh >= 0; --sh) {
+        const uint64_t blocks = ((n - 1) >> sh) + 1;
+        if (blocks > kMaxKeyBlocks) break;
+        bool wide = false;
+        const uint64_t b = threadIdx.x;
+        if (b < blocks) {
+            const uint64_t end = min(n, (b + 1) << sh);
+            wide = key[end - 1] - key[b << sh] > limit;
+        }
+        if (!__syncthreads_or(wide)) {
+            found = sh;
+            break;
+        }
+    }
+    if (threadIdx.x == 0) out[0] = found < 0 ? kNoKeyBlocks : static_cast<uint32_t>(found);
+    if (found >= 0 && threadIdx.x <= ((n - 1) >> found))
+        out[1 + threadIdx.x] = key[static_cast<uint64_t>(threadIdx.x) << found];
 }
 
 // Node-index entries: key = the list's node, value = the entry's walk record
@@ -529,8 +562,8 @@ __global__ __launch_bounds__(kB) void node_group_flags_packed_kernel(
 __global__ void node_group_scatter_kernel(const uint32_t* __restrict__ flags,
                                           const uint32_t* __restrict__ scan,
                                           const uint32_t* __restrict__ rank,
-                                          const int64_t* __restrict__ uniq_ts, size_t n,
-                                          uint32_t* __restrict__ grp,
+                                          const int64_t* __restrict__ uniq_ts, int time_keys,
+                                          int64_t t0, size_t n, uint32_t* __restrict__ grp,
                                           int64_t* __restrict__ first_ts,
                                           PanelRec* __restrict__ pan) {
     const size_t k = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
@@ -539,7 +572,7 @@ __global__ void node_group_scatter_kernel(const uint32_t* __restrict__ flags,
         const uint32_t g = scan[k];
         const uint32_t r = rank[k];
         grp[g] = static_cast<uint32_t>(k);
-        if (first_ts) first_ts[g] = uniq_ts[r];
+        if (first_ts) first_ts[g] = time_keys ? t0 + static_cast<int64_t>(r) : uniq_ts[r];
         pan[g] = PanelRec{r, static_cast<uint32_t>(k)};
     }
     if (k == n - 1) {
@@ -1270,7 +1303,7 @@ void build_direction(Engine& e, DirIndex& dir, size_t n, int key_bits, size_t vc
     // in 64 bits (cfg2: 20 + 25 + 17)
     const int nb = key_bits;
     const int eb = std::max(1, bit_length_u64(e.E ? e.E - 1 : 0));
-    const int rb = std::max(1, bit_length_u64(e.T ? e.T - 1 : 0));
+    const int rb = std::max(1, bit_length_u64(e.key_max));
     const bool packed = nb + eb + rb <= 64;
     dir.rec.resize(n);
     e.k32a.ensure(n);
@@ -1399,7 +1432,8 @@ void finish_direction(Engine& e, DirIndex& dir, size_t n, size_t vc, int64_t* ho
     dir.pan.resize(static_cast<size_t>(g) + 1);
     if (n) {
         hipLaunchKernelGGL(node_group_scatter_kernel, dim3(grid_for(n)), dim3(kB), 0, s,
-                           e.flags.p, e.scan.p, e.v32a.p, e.uniq_ts.p, n, dir.grp.p,
+                           e.flags.p, e.scan.p, e.v32a.p, e.uniq_ts.p, e.time_keys ? 1 : 0, e.key_t0, n,
+                           dir.grp.p,
                            weights ? dir.first_ts.p : nullptr, dir.pan.p);
     } else {
         check_hip(hipMemsetAsync(dir.grp.p, 0, 4, s), "grp terminator");
@@ -2030,12 +2064,33 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
     std::memcpy(&tg, hs + 1, 4);
     max_node_id = mx;
     T = tg;
+    const uint64_t range =
+        T ? static_cast<uint64_t>(store_tmax) - static_cast<uint64_t>(store_tmin) : 0;
+    time_keys = T > 0 && range <= kTimeKeyMax && range + 1 <= kTimeKeyGap * T;
+    key_t0 = store_tmin;
+    key_max = time_keys ? range : (T ? T - 1 : 0);
     tsg_off.resize(T + 1);
     uniq_ts.resize(T);
     erank.resize(E);
     hipLaunchKernelGGL(ts_group_scatter_kernel, dim3(grid_for(E)), dim3(kB), 0, s, ts.p, E,
-                       flags.p, scan.p, tsg_off.p, uniq_ts.p, erank.p);
+                       flags.p, scan.p, tsg_off.p, uniq_ts.p, time_keys ? 1 : 0, key_t0, erank.p);
     update_neg1_rank(*this);
+    check_hip(hipEventRecord(ts_ready, s), "event");
+
+    // ---- 5a. the key blocks of slot words that cannot hold a whole key, on
+    // the side stream (read by the walks only)
+    const int slot_bits = 64 - std::max(1, bit_length_u64(static_cast<uint64_t>(std::max(max_node_id, 0)))) -
+                          bit_length_u64(E ? E - 1 : 0);
+    const bool key_blocks = time_keys && slot_bits > 0 && slot_bits < bit_length_u64(key_max + 1);
+    kblk_shift = -1;
+    if (key_blocks) {
+        kblk.resize(1 + kMaxKeyBlocks);
+        check_hip(hipStreamWaitEvent(side, ts_ready, 0), "wait timestamp groups");
+        hipLaunchKernelGGL(key_block_table_kernel, dim3(1), dim3(1024), 0, side, erank.p,
+                           static_cast<uint64_t>(E), slot_bits, kblk.p);
+        check_hip(hipMemcpyAsync(hs + 8, kblk.p, 4, hipMemcpyDeviceToHost, side), "read key blocks");
+        check_hip(hipEventRecord(side_done, side), "event");
+    }
 
     // ---- 5b. global cumulative weights (edge_data.cu:440-514) on the side
     // stream, beside the node index: they read only the timestamp groups.
@@ -2044,7 +2099,6 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
     const bool weights = cfg.enable_weight_computation || cfg.enable_temporal_node2vec;
     if (weights) {
         hipStream_t sd = side;
-        check_hip(hipEventRecord(ts_ready, s), "event");
         check_hip(hipStreamWaitEvent(sd, ts_ready, 0), "wait timestamp groups");
         const double bound = cfg.timescale_bound;
         const double diff = static_cast<double>(store_tmax - store_tmin);
@@ -2204,6 +2258,11 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
     check_hip(hipStreamWaitEvent(s, side_done, 0), "wait side");
     check_hip(hipEventRecord(ev[3], s), "event");
     sync();
+    if (key_blocks) {
+        uint32_t sh;
+        std::memcpy(&sh, hs + 8, 4);
+        kblk_shift = sh == kNoKeyBlocks ? -1 : static_cast<int>(sh);
+    }
     float ms = 0;
     check_hip(hipEventElapsedTime(&ms, ev[0], ev[3]), "elapsed");
     timings.build_ms = ms;
@@ -2253,6 +2312,9 @@ void Engine::clear() {
     fwd_cum.n = bwd_cum.n = adj_off.n = adj_nbr.n = adj_hash.n = 0;
     gwg_fwd.n = gwg_bwd.n = gwt_fwd.n = gwt_bwd.n = 0;
     weights_ready = adj_ready = adj_lists_ready = false;
+    time_keys = false;
+    key_max = 0;
+    kblk_shift = -1;
     adj_nodes = 0;
     out.clear();
     in.clear();
@@ -2267,7 +2329,7 @@ void update_neg1_rank(Engine& e) {
 
 void launch_neg1_rank(Engine& e, int32_t* out) {
     hipLaunchKernelGGL(neg1_rank_kernel, dim3(1), dim3(1), 0, e.stream, e.uniq_ts.p,
-                       static_cast<uint32_t>(e.E ? e.T : 0), out);
+                       static_cast<uint32_t>(e.E ? e.T : 0), e.time_keys ? 1 : 0, e.key_t0, out);
     check_hip(hipGetLastError(), "neg1 rank launch");
 }
 

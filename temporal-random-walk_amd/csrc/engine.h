@@ -277,9 +277,18 @@ struct Engine {
     // timestamp groups
     DBuf<uint32_t> tsg_off;
     DBuf<int64_t> uniq_ts;
-    DBuf<uint32_t> erank;
-    DBuf<int32_t> neg1_rank;  // rank of timestamp -1 if stored, else -2
+    DBuf<uint32_t> erank;     // time key of every stored edge
+    DBuf<int32_t> neg1_rank;  // key of timestamp -1 if stored, else -2
     size_t T = 0;
+    // Time keys (index_layout.h): offsets from key_t0 (time_keys) or ranks,
+    // at most key_max; and, where a slot word cannot hold a whole key, its
+    // blocks (key_block_table_kernel): kblk[0] = shift or kNoKeyBlocks, then
+    // the first key of every block.  kblk_shift: its host copy, -1 for none.
+    bool time_keys = false;
+    int64_t key_t0 = 0;
+    uint64_t key_max = 0;
+    DBuf<uint32_t> kblk;
+    int kblk_shift = -1;
 
     // node map
     int32_t max_node_id = -1;

@@ -10,7 +10,7 @@
 //     src, dst      int32[E]      ts   int64[E]      feat fp32[E*dim]
 //   timestamp groups
 //     tsg_off       uint32[T+1]   uniq_ts int64[T]
-//     erank         uint32[E]     rank of every stored edge's timestamp
+//     erank         uint32[E]     time key of every stored edge (below)
 //   node map        active uint8[max_id+1]   (dense flags, as the reference)
 //   per direction (out = by source / both endpoints if undirected, in = by target)
 //     off           uint32[V_c]    CSR offsets, V_c = max_id + 2
@@ -68,6 +68,25 @@
 #include <stdint.h>
 
 namespace trw {
+
+// ---- time keys --------------------------------------------------------------
+// The index and the walks order times by a 32-bit key.  "Rank" in a name or a
+// comment here means this key.  It is the timestamp's rank among the graph's
+// unique timestamps, or -- where most time units of the store's span occur
+// (span + 1 <= kTimeKeyGap * unique timestamps) -- its offset from the store's
+// first timestamp.  Both order exactly as the timestamps do; the offset turns
+// back into the timestamp by an addition, the rank by a lookup in uniq_ts.
+// Gapped graphs keep ranks: their hubs then have a group at (nearly) every
+// key of their span, which the bucket tables answer without a search.
+constexpr uint64_t kTimeKeyGap = 2;
+constexpr uint64_t kTimeKeyMax = 0x7ffffff0ull;  // keys stay non-negative int32 values
+
+// Where node id, key and edge id do not fit in a 64-bit slot word together,
+// the word holds what the key exceeds the first key of the edge's block by (the
+// edges are sorted by time: a block is 2^shift consecutive edge ids): the
+// blocks' first keys are a table small enough for LDS.
+constexpr uint32_t kMaxKeyBlocks = 1024;
+constexpr uint32_t kNoKeyBlocks = 0xffffffffu;
 
 // One entry of a node's list as the walk reads it: the node reached over the
 // edge and the edge id, one 8-byte load.  Its timestamp is the
