@@ -361,8 +361,9 @@ struct Engine {
     DBuf<double> replay;
     // start-array temporaries of a sample (kept between calls: no per-call
     // allocation once they are large enough)
-    DBuf<int32_t> s_ids, s_seeds, s_tmp32;
-    DBuf<int64_t> s_cuts, s_tmp64;
+    DBuf<int32_t> s_ids, s_seeds;
+    DBuf<int64_t> s_cuts;
+    DBuf<uint8_t> s_flags;
     // node-grouped processing: walk states between segments, the (node, walk)
     // lists and the live count
     DBuf<uint32_t> ng_carry, ng_keys0, ng_keys1, ng_vals0, ng_vals1, ng_count;

@@ -1735,16 +1735,102 @@ __global__ __launch_bounds__(256) void layout_packed_kernel(LayoutArgs a) {
 }
 
 // ---- start arrays ----------------------------------------------------------
-__global__ void flags_from_u8_kernel(const uint8_t* __restrict__ a, size_t n,
-                                     uint32_t* __restrict__ f) {
-    const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i < n) f[i] = a[i] ? 1u : 0u;
+// The ascending ids whose flag byte is 1, kIdSpan ids per workgroup (16 per
+// thread, one 16-byte load): a count per workgroup, then every workgroup adds
+// the counts before its own (or finds them scanned, past kIdBlocks of them) and
+// writes its ids; the last one writes the total to pinned host memory.  A
+// graph of at most kIdSpan ids takes the second launch alone.
+constexpr uint32_t kIdSpan = kB * 16;
+constexpr size_t kIdBlocks = 2048;
+
+// The 16 flags from id i on (zeros past n).
+__device__ __forceinline__ void load_flags16(const uint8_t* __restrict__ f, size_t i, size_t n,
+                                             uint32_t (&w)[4]) {
+    w[0] = w[1] = w[2] = w[3] = 0u;
+    if (i + 16 <= n) {
+        const uint4 v = *reinterpret_cast<const uint4*>(f + i);
+        w[0] = v.x;
+        w[1] = v.y;
+        w[2] = v.z;
+        w[3] = v.w;
+    } else {
+        for (int k = 0; k < 16; ++k)
+            if (i + k < n) w[k >> 2] |= static_cast<uint32_t>(f[i + k]) << (8 * (k & 3));
+    }
 }
 
-__global__ void compact_ids_kernel(const uint32_t* __restrict__ f, const uint32_t* __restrict__ scan,
-                                   size_t n, int32_t* __restrict__ out) {
+__device__ __forceinline__ uint32_t flags16_count(const uint32_t (&w)[4]) {
+    return __popc(w[0]) + __popc(w[1]) + __popc(w[2]) + __popc(w[3]);
+}
+
+// Sum of v over the workgroup's threads before this one, and over all.
+__device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* total) {
+    __shared__ uint32_t s_wave[kB / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) s_wave[wave] = x;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < kB / 64; ++q) {
+        if (q < wave) before += s_wave[q];
+        all += s_wave[q];
+    }
+    __syncthreads();
+    *total = all;
+    return before + x - v;
+}
+
+__global__ __launch_bounds__(kB) void flag_counts_kernel(const uint8_t* __restrict__ f, size_t n,
+                                                         uint32_t* __restrict__ cnt) {
+    uint32_t w[4];
+    load_flags16(f, blockIdx.x * static_cast<size_t>(kIdSpan) + threadIdx.x * 16u, n, w);
+    uint32_t total;
+    (void)block_prefix(flags16_count(w), &total);
+    if (threadIdx.x == 0) cnt[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(kB) void flag_ids_kernel(const uint8_t* __restrict__ f, size_t n,
+                                                      const uint32_t* __restrict__ cnt, int scanned,
+                                                      int32_t* __restrict__ ids,
+                                                      uint32_t* __restrict__ total_out) {
+    uint32_t before = 0;
+    if (scanned) {
+        before = cnt[blockIdx.x];
+    } else if (blockIdx.x > 0) {
+        uint32_t mine = 0;
+        for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kB) mine += cnt[b];
+        (void)block_prefix(mine, &before);
+    }
+    const size_t i0 = blockIdx.x * static_cast<size_t>(kIdSpan) + threadIdx.x * 16u;
+    uint32_t w[4];
+    load_flags16(f, i0, n, w);
+    uint32_t total;
+    uint32_t at = before + block_prefix(flags16_count(w), &total);
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+        if ((w[k >> 2] >> (8 * (k & 3))) & 1u) ids[at++] = static_cast<int32_t>(i0 + k);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total_out = before + total;
+}
+
+// Flags (1) of the ids in a and, when given, b.
+__global__ __launch_bounds__(kB) void mark_ids_kernel(const int32_t* __restrict__ a,
+                                                      const int32_t* __restrict__ b, size_t n,
+                                                      uint8_t* __restrict__ f) {
     const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i < n && f[i]) out[scan[i]] = static_cast<int32_t>(i);
+    if (i >= n) return;
+    f[a[i]] = 1;
+    if (b) f[b[i]] = 1;
+}
+
+__global__ __launch_bounds__(kB) void clear_bytes_kernel(uint4* __restrict__ p, size_t n16) {
+    const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
+    if (i < n16) p[i] = uint4{0u, 0u, 0u, 0u};
 }
 
 __global__ void unique_flags_kernel(const uint32_t* __restrict__ k, size_t n,
@@ -1760,11 +1846,19 @@ __global__ void compact_keys_kernel(const uint32_t* __restrict__ k, const uint32
     if (i < n && f[i]) out[scan[i]] = static_cast<int32_t>(k[i]);
 }
 
-template <typename T>
-__global__ void repeat_kernel(const T* __restrict__ in, uint64_t n_out, int times,
-                              T* __restrict__ out) {
+// Every start id (and cutoff, when given) `times` over, in the order perm gives
+// (nullptr: as they come).
+__global__ __launch_bounds__(kB) void expand_starts_kernel(const int32_t* __restrict__ ids,
+                                                           const int64_t* __restrict__ cuts,
+                                                           const uint32_t* __restrict__ perm,
+                                                           uint64_t n_out, uint32_t times,
+                                                           int32_t* __restrict__ out,
+                                                           int64_t* __restrict__ out_cuts) {
     const uint64_t i = blockIdx.x * static_cast<uint64_t>(kB) + threadIdx.x;
-    if (i < n_out) out[i] = in[i / times];
+    if (i >= n_out) return;
+    const uint32_t k = (perm ? perm[i] : static_cast<uint32_t>(i)) / times;
+    out[i] = ids[k];
+    if (cuts) out_cuts[i] = cuts[k];
 }
 
 __global__ void random_keys_kernel(uint64_t n, uint32_t k0, uint32_t k1, uint32_t* __restrict__ keys,
@@ -1776,13 +1870,6 @@ __global__ void random_keys_kernel(uint64_t n, uint32_t k0, uint32_t k1, uint32_
                                k0, k1);
     keys[i] = o.x;
     vals[i] = static_cast<uint32_t>(i);
-}
-
-template <typename T>
-__global__ void permute_kernel(const T* __restrict__ in, const uint32_t* __restrict__ perm,
-                               uint64_t n, T* __restrict__ out) {
-    const uint64_t i = blockIdx.x * static_cast<uint64_t>(kB) + threadIdx.x;
-    if (i < n) out[i] = in[perm[i]];
 }
 
 __global__ void u32_from_i32_kernel(const int32_t* __restrict__ a, uint64_t n,
@@ -1974,6 +2061,9 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
     bool have_starts = false, have_cutoffs = false;
     int32_t* a_starts = nullptr;
     int64_t* a_cutoffs = nullptr;
+    const int32_t* start_ids = nullptr;   // the start nodes, wpn walks each
+    const int64_t* start_cuts = nullptr;  // and their cutoffs
+    auto bit_length = [](uint64_t v) { return v ? 64 - __builtin_clzll(v) : 0; };
     if (p.num_walks_per_node < 0 && p.mode != TRW_START_TOTAL)
         throw InvalidArgument("num_walks_per_node must be >= 0");
     const int wpn = p.num_walks_per_node;
@@ -1987,72 +2077,78 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
         }
         case TRW_START_ALL_NODES:
         case TRW_START_LAST_BATCH: {
+            // the active ids; or the unique sources (directed) or endpoints
+            // (undirected) of the last batch, ascending
+            // (core/temporal_random_walk.cu:157-272): from flags over its ids
+            // where those are no more than its entries, else from a sort
             size_t count = 0;
-            int32_t* ids = nullptr;
-            if (p.mode == TRW_START_ALL_NODES) {
-                const size_t v = active.n;
-                uint32_t* fl = sp.take(flags, v + 1);
-                uint32_t* sc = sp.take(scan, v + 1);
-                uint32_t* ss = sp.take(scan_scratch, scan_scratch_elems(v + 1));
-                if (v) {
-                    hipLaunchKernelGGL(flags_from_u8_kernel, dim3(grid_for(v)), dim3(kB), 0, s,
-                                       active.p, v, fl);
+            const size_t m = cfg.is_directed ? last_n : 2 * last_n;
+            const size_t batch_ids = last_n ? static_cast<size_t>(batch_max_id) + 1 : 0;
+            const bool all = p.mode == TRW_START_ALL_NODES;
+            if (all || batch_ids <= m) {
+                const size_t v = all ? active.n : batch_ids;
+                const uint8_t* fl = active.p;
+                if (!all && v) {
+                    const size_t n16 = (v + 15) / 16;
+                    uint8_t* f = sp.take(s_flags, 16 * n16);
+                    hipLaunchKernelGGL(clear_bytes_kernel, dim3(grid_for(n16)), dim3(kB), 0, s,
+                                       reinterpret_cast<uint4*>(f), n16);
+                    hipLaunchKernelGGL(mark_ids_kernel, dim3(grid_for(last_n)), dim3(kB), 0, s,
+                                       last_src.p, cfg.is_directed ? nullptr : last_dst.p, last_n, f);
+                    fl = f;
                 }
-                exclusive_scan_u32(fl, sc, v, ss, s);
-                check_hip(hipMemcpyAsync(hs, sc + v, 4, hipMemcpyDeviceToHost, s), "count");
-                sync();
-                uint32_t c;
-                std::memcpy(&c, hs, 4);
-                count = c;
-                ids = sp.take(s_ids, count);
+                const size_t nb = (v + kIdSpan - 1) / kIdSpan;
+                int32_t* out_ids = sp.take(s_ids, v);
                 if (v) {
-                    hipLaunchKernelGGL(compact_ids_kernel, dim3(grid_for(v)), dim3(kB), 0, s,
-                                       fl, sc, v, ids);
+                    const bool scanned = nb > kIdBlocks;
+                    uint32_t* cnt = sp.take(scan, nb + 1);
+                    if (nb > 1)
+                        hipLaunchKernelGGL(flag_counts_kernel, dim3(nb), dim3(kB), 0, s, fl, v, cnt);
+                    if (scanned)
+                        exclusive_scan_u32(cnt, cnt, nb,
+                                           sp.take(scan_scratch, scan_scratch_elems(nb)), s);
+                    // the total goes to the pinned scalars
+                    hipLaunchKernelGGL(flag_ids_kernel, dim3(nb), dim3(kB), 0, s, fl, v, cnt,
+                                       scanned ? 1 : 0, out_ids, reinterpret_cast<uint32_t*>(hs));
+                    check_hip(hipGetLastError(), "start ids launch");
+                    sync();
+                    uint32_t c;
+                    std::memcpy(&c, hs, 4);
+                    count = c;
                 }
+                start_ids = out_ids;
             } else {
-                // unique sources (directed) or unique endpoints (undirected) of the
-                // last batch, ascending (core/temporal_random_walk.cu:157-272)
-                const size_t m = cfg.is_directed ? last_n : 2 * last_n;
+                const int bits = std::max(1, bit_length(static_cast<uint64_t>(batch_max_id)));
                 uint32_t* ka = sp.take(k32a, m);
                 uint32_t* kb = sp.take(k32b, m);
-                const RadixTmp hi = sp.sort_tmp(hist, m, 32);
+                const RadixTmp hi = sp.sort_tmp(hist, m, bits);
                 uint32_t* fl = sp.take(flags, m + 1);
                 uint32_t* sc = sp.take(scan, m + 1);
                 uint32_t* ss = sp.take(scan_scratch, scan_scratch_elems(m + 1));
-                if (last_n) {
+                hipLaunchKernelGGL(u32_from_i32_kernel, dim3(grid_for(last_n)), dim3(kB), 0, s,
+                                   last_src.p, last_n, ka);
+                if (!cfg.is_directed) {
                     hipLaunchKernelGGL(u32_from_i32_kernel, dim3(grid_for(last_n)), dim3(kB), 0, s,
-                                       last_src.p, last_n, ka);
-                    if (!cfg.is_directed) {
-                        hipLaunchKernelGGL(u32_from_i32_kernel, dim3(grid_for(last_n)), dim3(kB),
-                                           0, s, last_dst.p, last_n, ka + last_n);
-                    }
+                                       last_dst.p, last_n, ka + last_n);
                 }
-                const int w = radix_sort_u32(ka, nullptr, kb, nullptr, m, 0, 32, hi, s);
+                const int w = radix_sort_u32(ka, nullptr, kb, nullptr, m, 0, bits, hi, s);
                 uint32_t* keys = w ? kb : ka;
-                if (m) {
-                    hipLaunchKernelGGL(unique_flags_kernel, dim3(grid_for(m)), dim3(kB), 0, s,
-                                       keys, m, fl);
-                }
+                hipLaunchKernelGGL(unique_flags_kernel, dim3(grid_for(m)), dim3(kB), 0, s, keys, m,
+                                   fl);
                 exclusive_scan_u32(fl, sc, m, ss, s);
                 check_hip(hipMemcpyAsync(hs, sc + m, 4, hipMemcpyDeviceToHost, s), "count");
                 sync();
                 uint32_t c;
                 std::memcpy(&c, hs, 4);
                 count = c;
-                ids = sp.take(s_ids, count);
-                if (m) {
-                    hipLaunchKernelGGL(compact_keys_kernel, dim3(grid_for(m)), dim3(kB), 0, s,
-                                       keys, fl, sc, m, ids);
-                }
+                int32_t* ids = sp.take(s_ids, count);
+                hipLaunchKernelGGL(compact_keys_kernel, dim3(grid_for(m)), dim3(kB), 0, s, keys, fl,
+                                   sc, m, ids);
+                start_ids = ids;
             }
             nw = static_cast<uint64_t>(count) * static_cast<uint64_t>(wpn);
             if (into && nw > into->capacity_walks)
                 throw InvalidArgument("the sample has more walks than the outputs' capacity");
-            a_starts = sp.take(starts, nw);
-            if (nw) {
-                hipLaunchKernelGGL((repeat_kernel<int32_t>), dim3(grid_for(nw)), dim3(kB), 0, s,
-                                   ids, nw, wpn, a_starts);
-            }
             have_starts = true;
             break;
         }
@@ -2067,11 +2163,7 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
                 check_hip(hipMemcpyAsync(seeds, p.seed_nodes, ns * 4, hipMemcpyHostToDevice, s),
                           "seeds H2D");
             }
-            a_starts = sp.take(starts, nw);
-            if (nw) {
-                hipLaunchKernelGGL((repeat_kernel<int32_t>), dim3(grid_for(nw)), dim3(kB), 0, s,
-                                   seeds, nw, wpn, a_starts);
-            }
+            start_ids = seeds;
             if (p.cutoff_times) {
                 int64_t* cuts = sp.take(s_cuts, ns);
                 if (ns) {
@@ -2079,11 +2171,7 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
                                              hipMemcpyHostToDevice, s),
                               "cutoffs H2D");
                 }
-                a_cutoffs = sp.take(cutoffs, nw);
-                if (nw) {
-                    hipLaunchKernelGGL((repeat_kernel<int64_t>), dim3(grid_for(nw)), dim3(kB), 0,
-                                       s, cuts, nw, wpn, a_cutoffs);
-                }
+                start_cuts = cuts;
                 have_cutoffs = true;
             }
             // the host arrays may be released once the copies have run
@@ -2097,27 +2185,29 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
     // one lane per walk: a dispatch holds fewer than 2^32 work-items
     if (nw >= (1ull << 32) - kB) throw InvalidArgument("too many walks (limit 2^32 - 256)");
 
-    // ---- optional shuffle of the walk order (same permutation for cutoffs)
-    if (have_starts && shuffle && nw > 1) {
-        if (nw > 0xffffffffull) throw InvalidArgument("shuffle supports < 2^32 walks");
-        uint32_t* ka = sp.take(k32a, nw);
-        uint32_t* kb = sp.take(k32b, nw);
-        uint32_t* va = sp.take(v32a, nw);
-        uint32_t* vb = sp.take(v32b, nw);
-        const RadixTmp hi = sp.sort_tmp(hist, nw, 32);
-        hipLaunchKernelGGL(random_keys_kernel, dim3(grid_for(nw)), dim3(kB), 0, s, nw,
-                           static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32), ka, va);
-        const int w = radix_sort_u32(ka, va, kb, vb, nw, 0, 32, hi, s);
-        const uint32_t* perm = w ? vb : va;
-        int32_t* ps = sp.take(s_tmp32, nw);
-        hipLaunchKernelGGL((permute_kernel<int32_t>), dim3(grid_for(nw)), dim3(kB), 0, s,
-                           a_starts, perm, nw, ps);
-        a_starts = ps;
-        if (have_cutoffs) {
-            int64_t* pc = sp.take(s_tmp64, nw);
-            hipLaunchKernelGGL((permute_kernel<int64_t>), dim3(grid_for(nw)), dim3(kB), 0, s,
-                               a_cutoffs, perm, nw, pc);
-            a_cutoffs = pc;
+    // ---- the walks' starts, with the optional shuffle of the walk order (same
+    // permutation for cutoffs)
+    if (have_starts) {
+        a_starts = sp.take(starts, nw);
+        if (have_cutoffs) a_cutoffs = sp.take(cutoffs, nw);
+        const uint32_t* perm = nullptr;
+        if (shuffle && nw > 1) {
+            if (nw > 0xffffffffull) throw InvalidArgument("shuffle supports < 2^32 walks");
+            uint32_t* ka = sp.take(k32a, nw);
+            uint32_t* kb = sp.take(k32b, nw);
+            uint32_t* va = sp.take(v32a, nw);
+            uint32_t* vb = sp.take(v32b, nw);
+            const RadixTmp hi = sp.sort_tmp(hist, nw, 32);
+            hipLaunchKernelGGL(random_keys_kernel, dim3(grid_for(nw)), dim3(kB), 0, s, nw,
+                               static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32), ka, va);
+            const int w = radix_sort_u32(ka, va, kb, vb, nw, 0, 32, hi, s);
+            perm = w ? vb : va;
+        }
+        if (nw) {
+            hipLaunchKernelGGL(expand_starts_kernel, dim3(grid_for(nw)), dim3(kB), 0, s, start_ids,
+                               start_cuts, perm, nw, static_cast<uint32_t>(wpn), a_starts,
+                               a_cutoffs);
+            check_hip(hipGetLastError(), "starts launch");
         }
     }
 
@@ -2154,7 +2244,6 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
     // for the first slot) and the id of the edge into the slot (below E), or,
     // when the three do not fit in 64 bits, node and edge id alone (rank
     // field width 0; the edge field's all-ones value marks the first slot)
-    auto bit_length = [](uint64_t v) { return v ? 64 - __builtin_clzll(v) : 0; };
     const int pk_nb = std::max(1, bit_length(static_cast<uint64_t>(std::max(max_node_id, 0))));
     const int rank_bits = bit_length(key_max + 1), eid_bits = E ? bit_length(E - 1) : 0;
     const bool with_rank = T > 0 && pk_nb + rank_bits + eid_bits <= 64;
