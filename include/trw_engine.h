@@ -240,6 +240,11 @@ trw_status trw_add_prefetched_edges(void* handle);
  * (core/temporal_random_walk.cu:657-916) and finalize_host_walks (:381-390):
  * outputs are copied to malloc'd host buffers owned by the caller. */
 trw_status trw_sample(void* handle, const trw_sample_params* params, trw_walks* out);
+/* Same; without edge ids (with_edge_ids 0) out->edge_ids is NULL and they are
+ * not copied to the host: two fifths of a walk set's bytes, for callers that
+ * have no use for them (the Python class returns none). */
+trw_status trw_sample_walks(void* handle, const trw_sample_params* params, int32_t with_edge_ids,
+                            trw_walks* out);
 /* Same, leaving the walks in device memory owned by the handle. */
 trw_status trw_sample_device(void* handle, const trw_sample_params* params, trw_walks* out);
 /* Same as trw_sample_device, into caller-owned device buffers, allocating

@@ -23,7 +23,9 @@ Engine::Engine(const trw_config& c) : cfg(c), device(c.device_id) {
     check_hip(hipEventCreateWithFlags(&side_done, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&ts_ready, hipEventDisableTiming), "hipEventCreate");
     for (auto& e : ev) check_hip(hipEventCreate(&e), "hipEventCreate");
-    check_hip(hipHostMalloc(&host_scalars, 256, hipHostMallocDefault), "hipHostMalloc");
+    check_hip(hipHostMalloc(&host_scalars, kScalarBytes + 12 * kMaxStagedSeeds, hipHostMallocDefault),
+              "hipHostMalloc");
+    attach_lanes(device);
 }
 
 Engine::~Engine() {
@@ -38,6 +40,7 @@ Engine::~Engine() {
     if (host_scalars) (void)hipHostFree(host_scalars);
     if (side) (void)hipStreamDestroy(side);
     if (stream) (void)hipStreamDestroy(stream);
+    detach_lanes(device);
 }
 
 size_t Engine::memory_used() const {
@@ -248,7 +251,7 @@ trw_status trw_prefetch_edges(void* handle, const int32_t* sources, const int32_
         e.pf_thread = std::thread([ep, segs]() {
             try {
                 trw::check_hip(hipSetDevice(ep->device), "hipSetDevice");
-                ep->copy_on_lanes(ep->pf_lanes, segs.data(), segs.size(), true, false);
+                ep->copy_on_lanes(segs.data(), segs.size(), true, false);
             } catch (const std::exception& ex) {
                 ep->pf_error = std::string("prefetch: ") + ex.what();
             }
@@ -333,6 +336,11 @@ trw_status trw_sample_device_noalloc(void* handle, const trw_sample_params* para
 }
 
 trw_status trw_sample(void* handle, const trw_sample_params* params, trw_walks* out) {
+    return trw_sample_walks(handle, params, 1, out);
+}
+
+trw_status trw_sample_walks(void* handle, const trw_sample_params* params, int32_t with_edge_ids,
+                            trw_walks* out) {
     return guarded(handle, [&](Engine& e) {
         if (!params || !out) throw trw::InvalidArgument("null argument");
         e.sample(*params);
@@ -352,7 +360,7 @@ trw_status trw_sample(void* handle, const trw_sample_params* params, trw_walks* 
             take(r.nodes, e.w_nodes.p, nw * L);
             take(r.timestamps, e.w_ts.p, nw * L);
             take(r.walk_lens, e.w_lens.p, nw);
-            take(r.edge_ids, e.w_eids.p, nw * el);
+            if (with_edge_ids) take(r.edge_ids, e.w_eids.p, nw * el);
             if (e.w_feat.n) {
                 r.feature_dim = static_cast<int32_t>(e.feat_dim);
                 take(r.edge_features, e.w_feat.p, e.w_feat.n);

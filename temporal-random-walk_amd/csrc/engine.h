@@ -238,7 +238,10 @@ struct HostCopy {
 };
 
 // Per-thread resources of the host handoff: a stream and two pinned staging
-// buffers (double buffering), created on first use.
+// buffers (double buffering), created on first use and kept in a pool per
+// device (handoff.hip) while the device has engines (attach / detach).
+void attach_lanes(int device);
+void detach_lanes(int device);
 struct HostLane {
     hipStream_t stream = nullptr;
     void* stage[2] = {nullptr, nullptr};
@@ -361,8 +364,8 @@ struct Engine {
     DBuf<double> replay;
     // start-array temporaries of a sample (kept between calls: no per-call
     // allocation once they are large enough)
-    DBuf<int32_t> s_ids, s_seeds;
-    DBuf<int64_t> s_cuts;
+    DBuf<int32_t> s_ids;
+    DBuf<int64_t> s_seeds;  // cutoffs, then seeds
     DBuf<uint8_t> s_flags;
     // node-grouped processing: walk states between segments, the (node, walk)
     // lists and the live count
@@ -391,15 +394,14 @@ struct Engine {
     int w_slot_format = 0;  // trw_walk_stats.slot_word_format of the last sample
     int w_replay = 0;
 
-    // pinned host scalars for the few readbacks that size allocations
+    // pinned host scalars for the few readbacks that size allocations, then
+    // room for a sample's seeds and cutoffs on their way to the device
     void* host_scalars = nullptr;
-
-    // host handoff lanes
-    std::vector<std::unique_ptr<HostLane>> lanes;
+    static constexpr size_t kScalarBytes = 256;
+    static constexpr size_t kMaxStagedSeeds = 4096;  // 12 bytes each
 
     // a host batch being staged into HBM beside other calls (trw_prefetch_edges):
-    // its own lanes and device buffers, and the thread that copies
-    std::vector<std::unique_ptr<HostLane>> pf_lanes;
+    // its own device buffers, and the thread that copies
     std::thread pf_thread;
     bool pf_pending = false;
     std::string pf_error;  // set by the copying thread on failure
@@ -459,11 +461,10 @@ struct Engine {
     // device (pinned staging, several threads); a device -> host copy records
     // timings.handoff_*.  Returns when every byte has landed.
     void copy_staged(const HostCopy* segs, size_t nseg, bool to_device);
-    // The same copy on the lanes ls, without waiting for the engine stream
-    // (small copies go through the first lane's stream): safe beside other
-    // work on the engine as long as no other call uses ls or the spans.
-    void copy_on_lanes(std::vector<std::unique_ptr<HostLane>>& ls, const HostCopy* segs, size_t nseg,
-                       bool to_device, bool engine_order);
+    // The same copy; without engine_order it does not wait for the engine
+    // stream (small copies go through a lane's own stream): safe beside other
+    // work on the engine as long as no other call uses the spans.
+    void copy_on_lanes(const HostCopy* segs, size_t nseg, bool to_device, bool engine_order);
     // Joins a pending prefetch; returns its error text ("" on success).
     std::string join_prefetch();
 };

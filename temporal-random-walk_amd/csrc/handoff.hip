@@ -10,9 +10,16 @@
 //    so first touch faults once per 2 MiB (they stay malloc-compatible:
 //    free() releases them, as the C ABI promises);
 //  - the copy is split into chunks that several host threads pull from one
-//    queue; each thread owns a HIP stream and two pinned staging buffers, so
-//    the DMA of its next chunk overlaps its memcpy of the current one, and
-//    the page faults of the destination are taken by all threads at once.
+//    queue; each thread owns a lane -- a HIP stream and two pinned staging
+//    buffers -- so the DMA of its next chunk overlaps its memcpy of the current
+//    one, and the page faults of the destination are taken by all threads at
+//    once; chunks shrink with the copy, so that a few MB still spread;
+//  - a copy of at most kPackBelow goes through one pinned buffer with one
+//    kernel on the engine's stream that moves every array (a runtime copy of
+//    pageable memory costs some 10 us per array): walks from 32 seeds 156 ->
+//    120 us.
+// Lanes are kept for the process in a pool per device: pinning their 16 MiB
+// takes longer than most copies, and a new handle need not pay it again.
 // Host-pointer ingest (trw_add_edges) uses the same lanes in the other
 // direction: the reference copies each batch array with one blocking
 // cudaMemcpy (data/buffer.cuh:135-149).
@@ -23,6 +30,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -35,8 +43,9 @@ namespace trw {
 namespace {
 
 constexpr size_t kHuge = size_t(2) << 20;
-constexpr size_t kChunk = size_t(8) << 20;          // bytes per staged chunk
-constexpr size_t kDirectBelow = size_t(32) << 20;   // smaller copies: one plain D2H
+constexpr size_t kChunk = size_t(8) << 20;        // bytes of a staging buffer
+constexpr size_t kMinChunk = size_t(512) << 10;   // smallest staged chunk
+constexpr size_t kPackBelow = size_t(2) << 20;    // smaller copies: one kernel
 constexpr int kMaxThreads = 32;
 
 int copy_threads() {
@@ -48,7 +57,83 @@ int copy_threads() {
     return n;
 }
 
+// The lanes not in use, per device.  At most kMaxThreads are kept on a device;
+// its last engine's end frees them.  (The pool itself is never destroyed:
+// nothing may call the runtime as the process ends.)
+struct LanePool {
+    struct Device {
+        std::vector<std::unique_ptr<HostLane>> free;
+        int engines = 0;
+    };
+    std::mutex mu;
+    std::map<int, Device> devices;
+};
+LanePool& lane_pool() {
+    static LanePool* pool = new LanePool;
+    return *pool;
+}
+
+// Lanes of the current device taken from the pool for one copy.
+struct Lanes {
+    int device;
+    std::vector<std::unique_ptr<HostLane>> v;
+    Lanes(int dev, int n) : device(dev) {
+        {
+            LanePool& p = lane_pool();
+            std::lock_guard<std::mutex> g(p.mu);
+            auto& f = p.devices[device].free;
+            while (static_cast<int>(v.size()) < n && !f.empty()) {
+                v.push_back(std::move(f.back()));
+                f.pop_back();
+            }
+        }
+        while (static_cast<int>(v.size()) < n) v.push_back(std::make_unique<HostLane>());
+    }
+    ~Lanes() {
+        LanePool& p = lane_pool();
+        std::lock_guard<std::mutex> g(p.mu);
+        auto& d = p.devices[device];
+        for (auto& l : v)
+            if (d.engines > 0 && d.free.size() < kMaxThreads) d.free.push_back(std::move(l));
+    }
+};
+
+// Up to kMaxSegs spans copied by one kernel, 16 bytes per thread: span i is the
+// units [at[i], at[i + 1]).  Every span starts 16-byte aligned on both sides.
+constexpr int kMaxSegs = 6;
+struct PackArgs {
+    const char* src[kMaxSegs];
+    char* dst[kMaxSegs];
+    uint64_t bytes[kMaxSegs];
+    uint64_t at[kMaxSegs + 1];
+    int n;
+};
+__global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
+    const uint64_t i = blockIdx.x * 256ull + threadIdx.x;
+    if (i >= a.at[a.n]) return;
+    int k = 0;
+    while (i >= a.at[k + 1]) ++k;
+    const uint64_t o = (i - a.at[k]) * 16;
+    if (o + 16 <= a.bytes[k]) {
+        *reinterpret_cast<uint4*>(a.dst[k] + o) = *reinterpret_cast<const uint4*>(a.src[k] + o);
+    } else {
+        for (uint64_t b = o; b < a.bytes[k]; ++b) a.dst[k][b] = a.src[k][b];
+    }
+}
+
 }  // namespace
+
+void attach_lanes(int device) {
+    std::lock_guard<std::mutex> g(lane_pool().mu);
+    ++lane_pool().devices[device].engines;
+}
+
+void detach_lanes(int device) {
+    std::vector<std::unique_ptr<HostLane>> done;
+    std::lock_guard<std::mutex> g(lane_pool().mu);
+    auto& d = lane_pool().devices[device];
+    if (--d.engines == 0) done.swap(d.free);
+}
 
 void* host_output_alloc(size_t bytes) {
     if (bytes < kHuge) {
@@ -73,14 +158,16 @@ HostLane::~HostLane() {
 }
 
 void HostLane::init() {
-    if (stream) return;
-    check_hip(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
-    for (auto& b : stage) check_hip(hipHostMalloc(&b, kChunk, hipHostMallocDefault), "hipHostMalloc");
-    for (auto& e : done) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    if (!stream)
+        check_hip(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
+    for (auto& b : stage)
+        if (!b) check_hip(hipHostMalloc(&b, kChunk, hipHostMallocDefault), "hipHostMalloc");
+    for (auto& e : done)
+        if (!e) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
 }
 
 void Engine::copy_staged(const HostCopy* segs, size_t nseg, bool to_device) {
-    copy_on_lanes(lanes, segs, nseg, to_device, true);
+    copy_on_lanes(segs, nseg, to_device, true);
 }
 
 std::string Engine::join_prefetch() {
@@ -92,37 +179,57 @@ std::string Engine::join_prefetch() {
     return err;
 }
 
-void Engine::copy_on_lanes(std::vector<std::unique_ptr<HostLane>>& ls, const HostCopy* segs,
-                           size_t nseg, bool to_device, bool engine_order) {
-    size_t total = 0;
-    for (size_t i = 0; i < nseg; ++i) total += segs[i].bytes;
+void Engine::copy_on_lanes(const HostCopy* segs, size_t nseg, bool to_device, bool engine_order) {
+    size_t total = 0, units = 0;
+    for (size_t i = 0; i < nseg; ++i) {
+        total += segs[i].bytes;
+        units += (segs[i].bytes + 15) / 16;
+    }
     // earlier work on the engine stream may still read or write these buffers
     if (engine_order) sync();
     const auto t0 = std::chrono::steady_clock::now();
-    const hipMemcpyKind kind = to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
 
-    if (total < kDirectBelow) {
-        hipStream_t st = stream;
-        if (!engine_order) {
-            if (ls.empty()) ls.push_back(std::make_unique<HostLane>());
-            ls[0]->init();
-            st = ls[0]->stream;
+    if (total == 0) {
+        // nothing to copy
+    } else if (units * 16 <= kPackBelow && nseg <= kMaxSegs) {
+        Lanes ls(device, 1);
+        ls.v[0]->init();
+        hipStream_t st = engine_order ? stream : ls.v[0]->stream;
+        char* stage = static_cast<char*>(ls.v[0]->stage[0]);
+        PackArgs a{};
+        for (size_t i = 0; i < nseg; ++i) {
+            if (!segs[i].bytes) continue;
+            char* at = stage + a.at[a.n] * 16;
+            if (to_device) memcpy(at, segs[i].src, segs[i].bytes);
+            a.src[a.n] = to_device ? at : static_cast<const char*>(segs[i].src);
+            a.dst[a.n] = to_device ? static_cast<char*>(segs[i].dst) : at;
+            a.bytes[a.n] = segs[i].bytes;
+            a.at[a.n + 1] = a.at[a.n] + (segs[i].bytes + 15) / 16;
+            ++a.n;
         }
-        for (size_t i = 0; i < nseg; ++i)
-            if (segs[i].bytes)
-                check_hip(hipMemcpyAsync(segs[i].dst, segs[i].src, segs[i].bytes, kind, st), "copy");
+        hipLaunchKernelGGL(pack_kernel, dim3(static_cast<unsigned>((units + 255) / 256)), dim3(256), 0,
+                           st, a);
+        check_hip(hipGetLastError(), "pack launch");
         check_hip(hipStreamSynchronize(st), "hipStreamSynchronize");
+        int k = 0;
+        for (size_t i = 0; i < nseg && !to_device; ++i) {
+            if (!segs[i].bytes) continue;
+            memcpy(segs[i].dst, a.dst[k++], segs[i].bytes);
+        }
     } else {
+        const size_t chunk_bytes = std::clamp(
+            (total / (2 * copy_threads()) + 65535) & ~size_t(65535), kMinChunk, kChunk);
         // chunk c of the whole transfer: segment seg_of[c], offset off_of[c]
         std::vector<size_t> seg_of, off_of;
         for (size_t i = 0; i < nseg; ++i)
-            for (size_t o = 0; o < segs[i].bytes; o += kChunk) {
+            for (size_t o = 0; o < segs[i].bytes; o += chunk_bytes) {
                 seg_of.push_back(i);
                 off_of.push_back(o);
             }
         const size_t nchunks = seg_of.size();
         const int nt = static_cast<int>(std::min<size_t>(copy_threads(), nchunks));
-        while (ls.size() < static_cast<size_t>(nt)) ls.push_back(std::make_unique<HostLane>());
+        Lanes taken(device, nt);
+        auto& ls = taken.v;
         for (int t = 0; t < nt; ++t) ls[t]->init();
 
         std::atomic<size_t> next{0};
@@ -131,7 +238,7 @@ void Engine::copy_on_lanes(std::vector<std::unique_ptr<HostLane>>& ls, const Hos
         std::string err;
         auto chunk = [&](size_t c, size_t* n) {
             const HostCopy& s = segs[seg_of[c]];
-            *n = std::min(kChunk, s.bytes - off_of[c]);
+            *n = std::min(chunk_bytes, s.bytes - off_of[c]);
             return s;
         };
         // device -> host: the DMA of a lane's next chunk into one staging

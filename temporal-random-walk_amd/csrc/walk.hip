@@ -2158,24 +2158,30 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
             nw = static_cast<uint64_t>(ns) * static_cast<uint64_t>(wpn);
             if (into && nw > into->capacity_walks)
                 throw InvalidArgument("the sample has more walks than the outputs' capacity");
-            int32_t* seeds = sp.take(s_seeds, ns);
-            if (ns) {
+            // cutoffs (when given), then seeds, in one buffer: through the
+            // pinned room beside the scalars in one copy that the call's end
+            // waits for, or -- past it -- copied from the caller's arrays
+            const size_t nc = p.cutoff_times ? ns : 0;
+            int64_t* buf = sp.take(s_seeds, nc + (ns + 1) / 2);
+            int32_t* seeds = reinterpret_cast<int32_t*>(buf + nc);
+            if (ns && ns <= kMaxStagedSeeds) {
+                char* stage = reinterpret_cast<char*>(hs) + kScalarBytes;
+                if (nc) std::memcpy(stage, p.cutoff_times, nc * 8);
+                std::memcpy(stage + nc * 8, p.seed_nodes, ns * 4);
+                check_hip(hipMemcpyAsync(buf, stage, nc * 8 + ns * 4, hipMemcpyHostToDevice, s),
+                          "seeds H2D");
+            } else if (ns) {
                 check_hip(hipMemcpyAsync(seeds, p.seed_nodes, ns * 4, hipMemcpyHostToDevice, s),
                           "seeds H2D");
+                if (nc)
+                    check_hip(hipMemcpyAsync(buf, p.cutoff_times, nc * 8, hipMemcpyHostToDevice, s),
+                              "cutoffs H2D");
+                // the host arrays may be released once the copies have run
+                sync();
             }
             start_ids = seeds;
-            if (p.cutoff_times) {
-                int64_t* cuts = sp.take(s_cuts, ns);
-                if (ns) {
-                    check_hip(hipMemcpyAsync(cuts, p.cutoff_times, ns * 8,
-                                             hipMemcpyHostToDevice, s),
-                              "cutoffs H2D");
-                }
-                start_cuts = cuts;
-                have_cutoffs = true;
-            }
-            // the host arrays may be released once the copies have run
-            sync();
+            have_cutoffs = p.cutoff_times != nullptr;
+            if (have_cutoffs) start_cuts = buf;
             have_starts = true;
             break;
         }

@@ -187,7 +187,7 @@ WalksWithEdgeFeaturesHost TemporalRandomWalk::sample(
     p.num_seed_nodes = num_seeds;
     p.shuffle = -1;
     trw_walks w{};
-    check(trw_sample(handle_, &p, &w));
+    check(trw_sample_walks(handle_, &p, with_edge_ids_ ? 1 : 0, &w));
     return WalksWithEdgeFeaturesHost(w);
 }
 

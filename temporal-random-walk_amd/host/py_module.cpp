@@ -123,7 +123,7 @@ PYBIND11_MODULE(_temporal_random_walk, m) {
                          std::optional<uint64_t> global_seed,
                          std::optional<bool> shuffle_walk_order,
                          std::optional<int> cuda_device_id) {
-                 return std::make_unique<TemporalRandomWalk>(
+                 auto tw = std::make_unique<TemporalRandomWalk>(
                      is_directed, use_gpu, max_time_capacity.value_or(-1),
                      enable_weight_computation.value_or(false),
                      enable_temporal_node2vec.value_or(false),
@@ -134,6 +134,8 @@ PYBIND11_MODULE(_temporal_random_walk, m) {
                      global_seed.value_or(EMPTY_GLOBAL_SEED),
                      shuffle_walk_order.value_or(DEFAULT_SHUFFLE_WALK_ORDER),
                      cuda_device_id.value_or(0));
+                 tw->set_with_edge_ids(false);  // walks_to_numpy returns none
+                 return tw;
              }),
              "Initialize a temporal random walk generator (runs on the MI355X; use_gpu is "
              "accepted for compatibility).",

@@ -65,6 +65,7 @@ ARRAYS = {
 EXPORTS = [
     "trw_create", "trw_destroy", "trw_last_error", "trw_abi_version", "trw_add_edges",
     "trw_add_edges_device", "trw_prefetch_edges", "trw_add_prefetched_edges", "trw_sample",
+    "trw_sample_walks",
     "trw_sample_device", "trw_sample_device_noalloc", "trw_walks_free",
     "trw_get_node_count", "trw_get_edge_count", "trw_get_node_ids", "trw_get_node_degrees",
     "trw_get_edges", "trw_get_is_directed", "trw_get_memory_used", "trw_get_feature_dim",
@@ -177,6 +178,8 @@ def lib():
         L.trw_prefetch_edges.argtypes = [P, P, P, P, C.c_uint64, P, C.c_uint64]
         L.trw_add_prefetched_edges.argtypes = [P]
         L.trw_sample.argtypes = [P, C.POINTER(TrwSampleParams), C.POINTER(TrwWalks)]
+        L.trw_sample_walks.argtypes = [P, C.POINTER(TrwSampleParams), C.c_int32,
+                                       C.POINTER(TrwWalks)]
         L.trw_sample_device.argtypes = [P, C.POINTER(TrwSampleParams), C.POINTER(TrwWalks)]
         L.trw_sample_device_noalloc.argtypes = [P, C.POINTER(TrwSampleParams), C.c_uint64,
                                                 C.POINTER(TrwWalks)]
