@@ -36,29 +36,22 @@ inline unsigned grid_for(size_t n) {
 
 inline int bit_length_u64(uint64_t v) { return v ? 64 - __builtin_clzll(v) : 0; }
 
-// Sort keys (ts - ts_min, 32-bit when the store's key range fits), positions,
-// and each edge's endpoints packed into one 8-byte word, so that the gather
-// after the sort costs one random load per edge instead of three.
+// Sort keys (ts - ts_min, 32-bit when the key range fits), positions, and each
+// edge's endpoints packed into one 8-byte word, so that the gather after the
+// sort costs one random load per edge instead of three: for batches with edge
+// features, whose sort carries positions (without them the sort reads the
+// batch itself, TsSource).
 template <typename K>
-__global__ void make_ts_keys_kernel(const int64_t* __restrict__ old_ts,
-                                    const int32_t* __restrict__ old_src,
-                                    const int32_t* __restrict__ old_dst, size_t e_old,
-                                    const int64_t* __restrict__ new_ts,
-                                    const int32_t* __restrict__ new_src,
-                                    const int32_t* __restrict__ new_dst, size_t n_new,
-                                    int64_t tmin, K* __restrict__ keys,
-                                    uint32_t* __restrict__ vals, uint64_t* __restrict__ ends) {
+__global__ void make_ts_keys_kernel(const int64_t* __restrict__ ts, const int32_t* __restrict__ src,
+                                    const int32_t* __restrict__ dst, size_t n, int64_t tmin,
+                                    K* __restrict__ keys, uint32_t* __restrict__ vals,
+                                    uint64_t* __restrict__ ends) {
     const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i >= e_old + n_new) return;
-    const bool old = i < e_old;
-    const size_t k = old ? i : i - e_old;
-    const int64_t t = old ? old_ts[k] : new_ts[k];
-    const int32_t a = old ? old_src[k] : new_src[k];
-    const int32_t b = old ? old_dst[k] : new_dst[k];
-    keys[i] = static_cast<K>(static_cast<uint64_t>(t) - static_cast<uint64_t>(tmin));
-    if (vals) vals[i] = static_cast<uint32_t>(i);
-    ends[i] = static_cast<uint64_t>(static_cast<uint32_t>(a)) |
-              (static_cast<uint64_t>(static_cast<uint32_t>(b)) << 32);
+    if (i >= n) return;
+    keys[i] = static_cast<K>(static_cast<uint64_t>(ts[i]) - static_cast<uint64_t>(tmin));
+    vals[i] = static_cast<uint32_t>(i);
+    ends[i] = static_cast<uint64_t>(static_cast<uint32_t>(src[i])) |
+              (static_cast<uint64_t>(static_cast<uint32_t>(dst[i])) << 32);
 }
 
 // out[0] = number of sorted keys <= target (upper_bound), out[1] = key at
@@ -156,29 +149,88 @@ inline unsigned grid_capped(size_t n) {
     return static_cast<unsigned>(g == 0 ? 1 : (g > (1u << 20) ? (1u << 20) : g));
 }
 
-__global__ void ts_group_flags_kernel(const int64_t* __restrict__ ts, size_t n,
-                                      uint32_t* __restrict__ flags) {
-    const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i >= n) return;
-    flags[i] = (i == 0 || ts[i] != ts[i - 1]) ? 1u : 0u;
+// ---- group starts (primitives.h) ---------------------------------------------
+// Each workgroup marks kGroupSpan positions: wave w its rows [8 w, 8 w + 8) of
+// 64, one word each.  start(i, row) tells whether position i < n starts a
+// group.  (The starts as one 32-bit flag per position, scanned into another
+// array in three launches, cost 6 passes over 4 bytes per position: at 20M
+// entries 110 us per direction that the bits take 25 us of.)
+constexpr int kSpanWaves = 4;
+constexpr int kSpanRows = static_cast<int>(kGroupSpan / 64 / kSpanWaves);
+static_assert(kSpanWaves * 64 == kB, "a span per workgroup");
+
+template <class Start>
+__device__ __forceinline__ void mark_groups(size_t n, uint64_t* __restrict__ bits,
+                                            uint32_t* __restrict__ spans, Start start) {
+    __shared__ uint32_t s_cnt[kSpanWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t base = blockIdx.x * kGroupSpan + static_cast<size_t>(wave) * kSpanRows * 64;
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int r = 0; r < kSpanRows; ++r) {
+        const size_t i = base + static_cast<size_t>(r) * 64 + lane;
+        const uint64_t m = __ballot(start(i, r));
+        if (lane == 0 && (i >> 6) < group_words(n)) bits[i >> 6] = m;
+        cnt += static_cast<uint32_t>(__popcll(m));
+    }
+    if (lane == 0) s_cnt[wave] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) spans[blockIdx.x] = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
 }
 
-__global__ void ts_group_scatter_kernel(const int64_t* __restrict__ ts, size_t n,
-                                        const uint32_t* __restrict__ flags,
-                                        const uint32_t* __restrict__ scan,
-                                        uint32_t* __restrict__ off, int64_t* __restrict__ uq,
-                                        int time_keys, int64_t t0,
-                                        uint32_t* __restrict__ erank) {
-    const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i >= n) return;
-    // the time key: the offset from the store's first timestamp, or the
-    // exclusive scan of the group-start flags: the group index of position i
-    erank[i] = time_keys ? static_cast<uint32_t>(ts[i] - t0) : scan[i] + flags[i] - 1u;
-    if (flags[i]) {
-        off[scan[i]] = static_cast<uint32_t>(i);
-        uq[scan[i]] = ts[i];
+// Calls f(i, group, starts) for the workgroup's positions i < n, group being
+// the number of groups that start before position i; spans scanned.
+template <class F>
+__device__ __forceinline__ void for_groups(size_t n, const uint64_t* __restrict__ bits,
+                                           const uint32_t* __restrict__ spans,
+                                           uint32_t* __restrict__ word_base, F f) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // lane w of every wave: the groups before word w of the span's 32
+    const size_t w0 = blockIdx.x * (kGroupSpan / 64);
+    const bool has = lane < static_cast<int>(kGroupSpan / 64) && w0 + lane < group_words(n);
+    const uint64_t word = has ? bits[w0 + lane] : 0ull;
+    const uint32_t c = static_cast<uint32_t>(__popcll(word));
+    uint32_t x = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
     }
-    if (i == n - 1) off[scan[n]] = static_cast<uint32_t>(n);
+    const uint32_t before = spans[blockIdx.x] + x - c;
+    if (word_base && wave == 0 && has) word_base[w0 + lane] = before;
+    const uint64_t below = lane ? ~0ull >> (64 - lane) : 0ull;
+#pragma unroll
+    for (int r = 0; r < kSpanRows; ++r) {
+        const int w = wave * kSpanRows + r;
+        const uint64_t m = __shfl(static_cast<unsigned long long>(word), w, 64);
+        const uint32_t b = __shfl(before, w, 64);
+        const size_t i = blockIdx.x * kGroupSpan + static_cast<size_t>(w) * 64 + lane;
+        if (i < n) f(i, b + static_cast<uint32_t>(__popcll(m & below)), ((m >> lane) & 1ull) != 0);
+    }
+}
+
+// Timestamp groups of the store.
+__global__ __launch_bounds__(kB) void ts_group_bits_kernel(const int64_t* __restrict__ ts, size_t n,
+                                                           uint64_t* __restrict__ bits,
+                                                           uint32_t* __restrict__ spans) {
+    mark_groups(n, bits, spans, [&](size_t i, int) {
+        return i < n && (i == 0 || ts[i] != ts[i - 1]);
+    });
+}
+
+__global__ __launch_bounds__(kB) void ts_group_scatter_kernel(
+    const int64_t* __restrict__ ts, size_t n, const uint64_t* __restrict__ bits,
+    const uint32_t* __restrict__ spans, uint32_t T, uint32_t* __restrict__ off,
+    int64_t* __restrict__ uq, int time_keys, int64_t t0, uint32_t* __restrict__ erank) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) off[T] = static_cast<uint32_t>(n);
+    for_groups(n, bits, spans, nullptr, [&](size_t i, uint32_t g, bool start) {
+        // the time key: the offset from the store's first timestamp, or the rank
+        erank[i] = time_keys ? static_cast<uint32_t>(ts[i] - t0) : g + (start ? 1u : 0u) - 1u;
+        if (start) {
+            off[g] = static_cast<uint32_t>(i);
+            uq[g] = ts[i];
+        }
+    });
 }
 
 // Key of timestamp -1, or -2 when no edge has it: the walk compares keys with
@@ -223,56 +275,6 @@ __global__ __launch_bounds__(1024) void key_block_table_kernel(const uint32_t* _
     if (threadIdx.x == 0) out[0] = found < 0 ? kNoKeyBlocks : static_cast<uint32_t>(found);
     if (found >= 0 && threadIdx.x <= ((n - 1) >> found))
         out[1 + threadIdx.x] = key[static_cast<uint64_t>(threadIdx.x) << found];
-}
-
-// Node-index entries: key = the list's node, value = the entry's walk record
-// (neighbour in the low word, edge id in the high word: EdgeRec's layout),
-// carried through the node sort so no record needs a gather afterwards.
-// mode 0: out-lists (node = source, neighbour = target); 1: in-lists (node =
-// target, neighbour = source); 2: undirected, entry 2i = (src_i; dst_i) and
-// entry 2i+1 = (dst_i; src_i) (node_edge_index.cu:306-321) -- the neighbour is
-// the reference's pick_other_number (utils/utils.cuh:102-104) seen from the
-// entry's node.
-__device__ __forceinline__ uint64_t pack_rec(int32_t nbr, uint32_t eid) {
-    return static_cast<uint64_t>(static_cast<uint32_t>(nbr)) | (static_cast<uint64_t>(eid) << 32);
-}
-
-// The edges are src/dst[0, e); their edge ids (store positions) start at id0.
-// With erank given, a value packs the neighbour, the edge id and the edge's
-// timestamp rank into one word (nbr | eid << nb | rank << (nb + eb); the caller
-// checks that they fit), so that the entries leave the node sort with their
-// ranks and the group flags need no gather of erank in node order.
-__global__ void node_entries_kernel(const int32_t* __restrict__ src,
-                                    const int32_t* __restrict__ dst, size_t e, int mode,
-                                    uint32_t id0, const uint32_t* __restrict__ erank, int nb,
-                                    int eb, uint32_t* __restrict__ keys,
-                                    uint64_t* __restrict__ vals) {
-    const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i >= e) return;
-    const int32_t a = src[i], b = dst[i];
-    const uint32_t id = id0 + static_cast<uint32_t>(i);
-    uint64_t va, vb;
-    if (erank) {
-        const uint64_t hi = (static_cast<uint64_t>(id) << nb) |
-                            (static_cast<uint64_t>(erank[id]) << (nb + eb));
-        va = hi | static_cast<uint32_t>(b);  // entry of a (out / first), neighbour b
-        vb = hi | static_cast<uint32_t>(a);
-    } else {
-        va = pack_rec(b, id);
-        vb = pack_rec(a, id);
-    }
-    if (mode == 0) {
-        keys[i] = static_cast<uint32_t>(a);
-        vals[i] = va;
-    } else if (mode == 1) {
-        keys[i] = static_cast<uint32_t>(b);
-        vals[i] = vb;
-    } else {
-        keys[2 * i] = static_cast<uint32_t>(a);
-        vals[2 * i] = va;
-        keys[2 * i + 1] = static_cast<uint32_t>(b);
-        vals[2 * i + 1] = vb;
-    }
 }
 
 // off[u] = first sorted position whose node >= u, u in [0, vc).
@@ -508,86 +510,126 @@ __global__ void merge_new_kernel(const int64_t* __restrict__ old_ts, size_t del_
     if (perm) perm[p] = static_cast<uint32_t>(e_old) + bpos[j];
 }
 
-// Group-start flags of the sorted entries (a new node, or a new timestamp
-// rank within a node) and the sorted edge ids (node_ts_sorted_*_indices).  The
-// previous entry's node and rank come from the lane below.
-__global__ __launch_bounds__(kB) void node_group_flags_kernel(const uint32_t* __restrict__ keys,
-                                                              const EdgeRec* __restrict__ rec,
-                                                              const uint32_t* __restrict__ erank,
-                                                              size_t n,
-                                                              uint32_t* __restrict__ flags,
-                                                              uint32_t* __restrict__ idx,
-                                                              uint32_t* __restrict__ rank) {
-    const size_t k = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (k >= n) return;  // the active lanes of a wave are a prefix
-    const uint32_t key = keys[k];
-    const uint32_t e = rec[k].eid;
-    const uint32_t r = erank[e];
-    idx[k] = e;
-    rank[k] = r;
-    uint32_t kp = __shfl_up(key, 1, 64), rp = __shfl_up(r, 1, 64);
-    if ((threadIdx.x & 63) == 0 && k > 0) {
-        kp = keys[k - 1];
-        rp = erank[rec[k - 1].eid];
+// Group starts of the sorted entries (a new node, or a new timestamp rank within
+// a node), the sorted edge ids (node_ts_sorted_*_indices) and the entries'
+// ranks.  The previous entry's node and rank come from the lane below, or from
+// the wave's row above.
+__global__ __launch_bounds__(kB) void node_group_bits_kernel(const uint32_t* __restrict__ keys,
+                                                             const EdgeRec* __restrict__ rec,
+                                                             const uint32_t* __restrict__ erank,
+                                                             size_t n, uint64_t* __restrict__ bits,
+                                                             uint32_t* __restrict__ spans,
+                                                             uint32_t* __restrict__ idx,
+                                                             uint32_t* __restrict__ rank) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t base = blockIdx.x * kGroupSpan + static_cast<size_t>(wave) * kSpanRows * 64;
+    uint32_t key[kSpanRows], e[kSpanRows], rk[kSpanRows];
+#pragma unroll
+    for (int r = 0; r < kSpanRows; ++r) {
+        const size_t k = base + static_cast<size_t>(r) * 64 + lane;
+        key[r] = k < n ? keys[k] : 0u;
+        e[r] = k < n ? rec[k].eid : 0u;
     }
-    flags[k] = (k == 0 || key != kp || r != rp) ? 1u : 0u;
+#pragma unroll
+    for (int r = 0; r < kSpanRows; ++r) {
+        const size_t k = base + static_cast<size_t>(r) * 64 + lane;
+        rk[r] = k < n ? erank[e[r]] : 0u;
+        if (k < n) {
+            idx[k] = e[r];
+            rank[k] = rk[r];
+        }
+    }
+    uint32_t above_k = 0, above_r = 0;  // the entry before the wave's first
+    if (base > 0 && base < n) {
+        above_k = keys[base - 1];
+        above_r = erank[rec[base - 1].eid];
+    }
+    mark_groups(n, bits, spans, [&](size_t k, int r) {
+        uint32_t kp = __shfl_up(key[r], 1, 64), rp = __shfl_up(rk[r], 1, 64);
+        if (lane == 0) {
+            kp = above_k;
+            rp = above_r;
+        }
+        above_k = __shfl(key[r], 63, 64);
+        above_r = __shfl(rk[r], 63, 64);
+        return k < n && (k == 0 || key[r] != kp || rk[r] != rp);
+    });
 }
 
-// node_group_flags_kernel for entries whose sorted values carry their ranks
-// (node_entries_kernel with erank): also unpacks the walk records.
-__global__ __launch_bounds__(kB) void node_group_flags_packed_kernel(
+// node_group_bits_kernel for entries whose sorted values carry their ranks
+// (EntrySource with erank): also unpacks the walk records.  rank: written when
+// given (the weights' records need every entry's).
+__global__ __launch_bounds__(kB) void node_group_bits_packed_kernel(
     const uint32_t* __restrict__ keys, const uint64_t* __restrict__ packed, size_t n, int nb,
-    int eb, uint32_t* __restrict__ flags, uint32_t* __restrict__ idx,
+    int eb, uint64_t* __restrict__ bits, uint32_t* __restrict__ spans, uint32_t* __restrict__ idx,
     uint32_t* __restrict__ rank, EdgeRec* __restrict__ rec) {
-    const size_t k = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (k >= n) return;  // the active lanes of a wave are a prefix
-    const uint32_t key = keys[k];
-    const uint64_t v = packed[k];
-    const uint32_t e = static_cast<uint32_t>((v >> nb) & ((1ull << eb) - 1ull));
-    const uint32_t r = static_cast<uint32_t>(v >> (nb + eb));
-    rec[k] = EdgeRec{static_cast<int32_t>(static_cast<uint32_t>(v & ((1ull << nb) - 1ull))), e};
-    idx[k] = e;
-    rank[k] = r;
-    uint32_t kp = __shfl_up(key, 1, 64), rp = __shfl_up(r, 1, 64);
-    if ((threadIdx.x & 63) == 0 && k > 0) {
-        kp = keys[k - 1];
-        rp = static_cast<uint32_t>(packed[k - 1] >> (nb + eb));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t base = blockIdx.x * kGroupSpan + static_cast<size_t>(wave) * kSpanRows * 64;
+    uint32_t key[kSpanRows], rk[kSpanRows];
+#pragma unroll
+    for (int r = 0; r < kSpanRows; ++r) {
+        const size_t k = base + static_cast<size_t>(r) * 64 + lane;
+        key[r] = k < n ? keys[k] : 0u;
+        const uint64_t v = k < n ? packed[k] : 0ull;
+        const uint32_t e = static_cast<uint32_t>((v >> nb) & ((1ull << eb) - 1ull));
+        rk[r] = static_cast<uint32_t>(v >> (nb + eb));
+        if (k < n) {
+            rec[k] = EdgeRec{static_cast<int32_t>(static_cast<uint32_t>(v & ((1ull << nb) - 1ull))),
+                             e};
+            idx[k] = e;
+            if (rank) rank[k] = rk[r];
+        }
     }
-    flags[k] = (k == 0 || key != kp || r != rp) ? 1u : 0u;
+    uint32_t above_k = 0, above_r = 0;  // the entry before the wave's first
+    if (base > 0 && base < n) {
+        above_k = keys[base - 1];
+        above_r = static_cast<uint32_t>(packed[base - 1] >> (nb + eb));
+    }
+    mark_groups(n, bits, spans, [&](size_t k, int r) {
+        uint32_t kp = __shfl_up(key[r], 1, 64), rp = __shfl_up(rk[r], 1, 64);
+        if (lane == 0) {
+            kp = above_k;
+            rp = above_r;
+        }
+        above_k = __shfl(key[r], 63, 64);
+        above_r = __shfl(rk[r], 63, 64);
+        return k < n && (k == 0 || key[r] != kp || rk[r] != rp);
+    });
 }
 
 // Group starts, panel records and (for the weights, when first_ts is given)
-// each group's timestamp, from the flags, their scan and the entries' ranks
-// (all read in entry order).
-__global__ void node_group_scatter_kernel(const uint32_t* __restrict__ flags,
-                                          const uint32_t* __restrict__ scan,
-                                          const uint32_t* __restrict__ rank,
-                                          const int64_t* __restrict__ uniq_ts, int time_keys,
-                                          int64_t t0, size_t n, uint32_t* __restrict__ grp,
-                                          int64_t* __restrict__ first_ts,
-                                          PanelRec* __restrict__ pan) {
-    const size_t k = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (k >= n) return;
-    if (flags[k]) {
-        const uint32_t g = scan[k];
-        const uint32_t r = rank[k];
+// each group's timestamp, from the start bits and the entries' ranks (rank, or
+// packed >> shift).  word_base: the groups before every word of bits.
+__global__ __launch_bounds__(kB) void node_group_scatter_kernel(
+    const uint64_t* __restrict__ bits, const uint32_t* __restrict__ spans,
+    uint32_t* __restrict__ word_base, const uint32_t* __restrict__ rank,
+    const uint64_t* __restrict__ packed, int shift, const int64_t* __restrict__ uniq_ts,
+    int time_keys, int64_t t0, size_t n, uint32_t g_all, uint32_t* __restrict__ grp,
+    int64_t* __restrict__ first_ts, PanelRec* __restrict__ pan) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        grp[g_all] = static_cast<uint32_t>(n);
+        pan[g_all] = PanelRec{n ? 0xffffffffu : 0u, static_cast<uint32_t>(n)};
+    }
+    for_groups(n, bits, spans, word_base, [&](size_t k, uint32_t g, bool start) {
+        if (!start) return;
+        const uint32_t r = rank ? rank[k] : static_cast<uint32_t>(packed[k] >> shift);
         grp[g] = static_cast<uint32_t>(k);
         if (first_ts) first_ts[g] = time_keys ? t0 + static_cast<int64_t>(r) : uniq_ts[r];
         pan[g] = PanelRec{r, static_cast<uint32_t>(k)};
-    }
-    if (k == n - 1) {
-        grp[scan[n]] = static_cast<uint32_t>(n);
-        pan[scan[n]] = PanelRec{0xffffffffu, static_cast<uint32_t>(n)};
-    }
+    });
 }
 
-// cnt[u] = number of groups of nodes < u = flag scan at u's first entry.
+// cnt[u] = number of groups of nodes < u: those that start before u's first
+// entry.
 __global__ void node_group_counts_kernel(const uint32_t* __restrict__ off,
-                                         const uint32_t* __restrict__ scan, size_t vc,
+                                         const uint64_t* __restrict__ bits,
+                                         const uint32_t* __restrict__ word_base, size_t vc,
                                          uint32_t* __restrict__ cnt) {
     const size_t u = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
     if (u >= vc) return;
-    cnt[u] = scan[off[u]];
+    const uint32_t o = off[u];
+    const uint64_t below = (1ull << (o & 63u)) - 1ull;
+    cnt[u] = word_base[o >> 6] + static_cast<uint32_t>(__popcll(bits[o >> 6] & below));
 }
 
 // Bucket shift of a node with G > kTabMin groups whose ranks span `span`:
@@ -975,10 +1017,12 @@ __global__ void adj_pair_keys_kernel(const int32_t* __restrict__ s, const int32_
     keys[i] = (min(u, v) << b) | max(u, v);
 }
 
-__global__ void distinct_flags_kernel(const uint32_t* __restrict__ keys, size_t n,
-                                      uint32_t* __restrict__ flags) {
-    const size_t i = blockIdx.x * static_cast<size_t>(kB) + threadIdx.x;
-    if (i < n) flags[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1u : 0u;
+__global__ __launch_bounds__(kB) void distinct_bits_kernel(const uint32_t* __restrict__ keys,
+                                                           size_t n, uint64_t* __restrict__ bits,
+                                                           uint32_t* __restrict__ spans) {
+    mark_groups(n, bits, spans, [&](size_t i, int) {
+        return i < n && (i == 0 || keys[i] != keys[i - 1]);
+    });
 }
 
 // Global per-timestamp-group weights before normalisation
@@ -1282,7 +1326,7 @@ void validate_batch(const Engine& e, const void* feat, size_t n, size_t dim) {
 namespace {
 
 // Sorted node-index entries whose values carry their timestamp ranks
-// (node_entries_kernel with erank), or none (vals == nullptr: dir.rec holds
+// (EntrySource with erank), or none (vals == nullptr: dir.rec holds
 // the records and the ranks are gathered from erank).
 struct PackedEntries {
     const uint64_t* vals;
@@ -1293,7 +1337,7 @@ void finish_direction(Engine& e, DirIndex& dir, size_t n, size_t vc, int64_t* ho
                       const PackedEntries& pe);
 
 // Stable per-direction node index of the store's n entries (mode: see
-// node_entries_kernel).
+// EntrySource).
 void build_direction(Engine& e, DirIndex& dir, size_t n, int key_bits, size_t vc, int mode,
                      int64_t* host_scratch) {
     hipStream_t s = e.stream;
@@ -1316,12 +1360,8 @@ void build_direction(Engine& e, DirIndex& dir, size_t n, int key_bits, size_t vc
     uint64_t* recs = reinterpret_cast<uint64_t*>(dir.rec.p);
     uint64_t* v0 = packed ? e.k64a.p : (passes % 2 == 0 ? recs : e.k64a.p);
     uint64_t* v1 = packed ? e.k64b.p : (passes % 2 == 0 ? e.k64a.p : recs);
-    const size_t edges = mode == 2 ? n / 2 : n;
-    if (edges)
-        hipLaunchKernelGGL(node_entries_kernel, dim3(grid_for(edges)), dim3(kB), 0, s, e.src.p,
-                           e.dst.p, edges, mode, 0u, packed ? e.erank.p : nullptr, nb, eb,
-                           e.k32a.p, v0);
-    const int which = radix_sort_u32_v64(e.k32a.p, v0, e.k32b.p, v1, n, 0, key_bits,
+    const EntrySource in{e.src.p, e.dst.p, mode, 0u, packed ? e.erank.p : nullptr, nb, eb};
+    const int which = radix_sort_entries(in, e.k32a.p, v0, e.k32b.p, v1, n, key_bits,
                                          e.radix_tmp(n, key_bits), s);
     // the sorted keys become the direction's (the scratch takes the old
     // buffer, which every user sizes again before writing)
@@ -1339,7 +1379,7 @@ void build_direction(Engine& e, DirIndex& dir, size_t n, int key_bits, size_t vc
 // lowered by the evicted count), then its batch entries in batch order -- the
 // stable (node, position) order of the new store, because the kept old edges
 // precede the batch.  Only the batch's entries are sorted; the old entries
-// move by one scatter.  mode as node_entries_kernel.
+// move by one scatter.  mode as EntrySource.
 void append_direction(Engine& e, DirIndex& dir, int mode, int key_bits, size_t vc,
                       int64_t* host_scratch) {
     hipStream_t s = e.stream;
@@ -1358,11 +1398,8 @@ void append_direction(Engine& e, DirIndex& dir, int mode, int key_bits, size_t v
     e.k64a.ensure(m);
     e.k64b.ensure(m);
     const uint32_t id0 = static_cast<uint32_t>(e.append_kept_old);
-    if (e.append_kept_new)
-        hipLaunchKernelGGL(node_entries_kernel, dim3(grid_for(e.append_kept_new)), dim3(kB), 0, s,
-                           e.src.p + id0, e.dst.p + id0, e.append_kept_new, mode, id0, nullptr, 0,
-                           0, e.k32a.p, e.k64a.p);
-    const int w = radix_sort_u32_v64(e.k32a.p, e.k64a.p, e.k32b.p, e.k64b.p, m, 0, key_bits,
+    const EntrySource in{e.src.p + id0, e.dst.p + id0, mode, id0, nullptr, 0, 0};
+    const int w = radix_sort_entries(in, e.k32a.p, e.k64a.p, e.k32b.p, e.k64b.p, m, key_bits,
                                      e.radix_tmp(m, key_bits), s);
     const uint32_t* bkeys = w ? e.k32b.p : e.k32a.p;
     const uint64_t* brec = w ? e.k64b.p : e.k64a.p;
@@ -1411,37 +1448,39 @@ void finish_direction(Engine& e, DirIndex& dir, size_t n, size_t vc, int64_t* ho
                       const PackedEntries& pe) {
     hipStream_t s = e.stream;
     dir.idx.resize(n);
-    e.v32a.ensure(n);  // the entries' timestamp ranks
+    // group timestamps feed only the per-node weights, and every entry's
+    // timestamp rank only their records (and entries that carry none)
+    const bool weights = e.cfg.enable_weight_computation || e.cfg.enable_temporal_node2vec;
+    uint32_t* rank = nullptr;
+    if (weights || !pe.vals) {
+        e.v32a.ensure(n);
+        rank = e.v32a.p;
+    }
+    const unsigned spans = static_cast<unsigned>(group_spans(n));
+    e.gbits.ensure(group_words(n));
+    e.gwords.ensure(group_words(n));
+    e.gspans.ensure(spans);
     if (pe.vals)
-        hipLaunchKernelGGL(node_group_flags_packed_kernel, dim3(grid_for(n)), dim3(kB), 0, s,
-                           dir.key.p, pe.vals, n, pe.nb, pe.eb, e.flags.p, dir.idx.p, e.v32a.p,
+        hipLaunchKernelGGL(node_group_bits_packed_kernel, dim3(spans), dim3(kB), 0, s, dir.key.p,
+                           pe.vals, n, pe.nb, pe.eb, e.gbits.p, e.gspans.p, dir.idx.p, rank,
                            dir.rec.p);
     else
-        hipLaunchKernelGGL(node_group_flags_kernel, dim3(grid_for(n)), dim3(kB), 0, s, dir.key.p,
-                           dir.rec.p, e.erank.p, n, e.flags.p, dir.idx.p, e.v32a.p);
-    exclusive_scan_u32(e.flags.p, e.scan.p, n, e.scan_scratch.p, s);
-    uint32_t g = 0;
-    check_hip(hipMemcpyAsync(host_scratch, e.scan.p + n, 4, hipMemcpyDeviceToHost, s), "read g");
+        hipLaunchKernelGGL(node_group_bits_kernel, dim3(spans), dim3(kB), 0, s, dir.key.p,
+                           dir.rec.p, e.erank.p, n, e.gbits.p, e.gspans.p, dir.idx.p, rank);
+    group_scan(e.gspans.p, spans, reinterpret_cast<uint32_t*>(host_scratch), s);
     e.sync();
+    uint32_t g = 0;
     std::memcpy(&g, host_scratch, 4);
     dir.n_groups = g;
     dir.grp.resize(static_cast<size_t>(g) + 1);
-    // group timestamps feed only the per-node weights
-    const bool weights = e.cfg.enable_weight_computation || e.cfg.enable_temporal_node2vec;
     dir.first_ts.resize(weights ? g : 0);
     dir.pan.resize(static_cast<size_t>(g) + 1);
-    if (n) {
-        hipLaunchKernelGGL(node_group_scatter_kernel, dim3(grid_for(n)), dim3(kB), 0, s,
-                           e.flags.p, e.scan.p, e.v32a.p, e.uniq_ts.p, e.time_keys ? 1 : 0, e.key_t0, n,
-                           dir.grp.p,
-                           weights ? dir.first_ts.p : nullptr, dir.pan.p);
-    } else {
-        check_hip(hipMemsetAsync(dir.grp.p, 0, 4, s), "grp terminator");
-        check_hip(hipMemsetAsync(dir.pan.p, 0, sizeof(PanelRec), s), "panel terminator");
-    }
+    hipLaunchKernelGGL(node_group_scatter_kernel, dim3(spans), dim3(kB), 0, s, e.gbits.p, e.gspans.p,
+                       e.gwords.p, rank, pe.vals, pe.nb + pe.eb, e.uniq_ts.p, e.time_keys ? 1 : 0,
+                       e.key_t0, n, g, dir.grp.p, weights ? dir.first_ts.p : nullptr, dir.pan.p);
     dir.cnt.resize(vc);
     hipLaunchKernelGGL(node_group_counts_kernel, dim3(grid_for(vc)), dim3(kB), 0, s, dir.off.p,
-                       e.scan.p, vc, dir.cnt.p);
+                       e.gbits.p, e.gwords.p, vc, dir.cnt.p);
 
     // walk search headers and bucket tables
     dir.hdr.resize(vc);
@@ -1583,6 +1622,25 @@ struct SortedBatch {
     const uint32_t* bpos;
 };
 
+// The sort of a batch with edge features: positions (v32a / v32b) by timestamp
+// (k64a / k64b, 32-bit keys when `bits` fit), the packed endpoints in batch
+// order beside them (ends64).
+int sort_positions(Engine& e, const int32_t* d_src, const int32_t* d_dst, const int64_t* d_ts,
+                   size_t n, int64_t tmin, int bits, RadixTmp tmp) {
+    hipStream_t s = e.stream;
+    e.v32a.ensure(n);
+    e.v32b.ensure(n);
+    if (bits <= 32) {
+        uint32_t* k[2] = {reinterpret_cast<uint32_t*>(e.k64a.p), reinterpret_cast<uint32_t*>(e.k64b.p)};
+        hipLaunchKernelGGL((make_ts_keys_kernel<uint32_t>), dim3(grid_for(n)), dim3(kB), 0, s, d_ts,
+                           d_src, d_dst, n, tmin, k[0], e.v32a.p, e.ends64.p);
+        return radix_sort_u32(k[0], e.v32a.p, k[1], e.v32b.p, n, 0, bits, tmp, s);
+    }
+    hipLaunchKernelGGL((make_ts_keys_kernel<uint64_t>), dim3(grid_for(n)), dim3(kB), 0, s, d_ts, d_src,
+                       d_dst, n, tmin, e.k64a.p, e.v32a.p, e.ends64.p);
+    return radix_sort_u64(e.k64a.p, e.v32a.p, e.k64b.p, e.v32b.p, n, 0, bits, tmp, s);
+}
+
 SortedBatch sort_batch(Engine& e, const int32_t* d_src, const int32_t* d_dst, const int64_t* d_ts,
                        size_t n, int64_t btmin, int64_t btmax) {
     hipStream_t s = e.stream;
@@ -1593,28 +1651,17 @@ SortedBatch sort_batch(Engine& e, const int32_t* d_src, const int32_t* d_dst, co
     e.k64b.ensure(n);
     e.ends64.ensure(n);
     if (carry_ends) e.ends64b.ensure(n);
-    e.v32a.ensure(n);
-    e.v32b.ensure(n);
     const RadixTmp tmp = e.radix_tmp(n, bits);
     uint32_t* k32s[2] = {reinterpret_cast<uint32_t*>(e.k64a.p), reinterpret_cast<uint32_t*>(e.k64b.p)};
-    uint32_t* pos0 = carry_ends ? nullptr : e.v32a.p;
     int which;
-    if (keys32) {
-        hipLaunchKernelGGL((make_ts_keys_kernel<uint32_t>), dim3(grid_for(n)), dim3(kB), 0, s,
-                           e.ts.p, e.src.p, e.dst.p, size_t{0}, d_ts, d_src, d_dst, n, btmin,
-                           k32s[0], pos0, e.ends64.p);
-        which = carry_ends ? radix_sort_u32_v64(k32s[0], e.ends64.p, k32s[1], e.ends64b.p, n, 0,
-                                                bits, tmp, s)
-                           : radix_sort_u32(k32s[0], e.v32a.p, k32s[1], e.v32b.p, n, 0, bits,
-                                            tmp, s);
+    if (carry_ends) {
+        const TsSource in{d_ts, d_src, d_dst, btmin};
+        which = keys32 ? radix_sort_ts_u32(in, k32s[0], e.ends64.p, k32s[1], e.ends64b.p, n, bits, tmp,
+                                           s, nullptr)
+                       : radix_sort_ts_u64(in, e.k64a.p, e.ends64.p, e.k64b.p, e.ends64b.p, n, bits,
+                                           tmp, s, nullptr);
     } else {
-        hipLaunchKernelGGL((make_ts_keys_kernel<uint64_t>), dim3(grid_for(n)), dim3(kB), 0, s,
-                           e.ts.p, e.src.p, e.dst.p, size_t{0}, d_ts, d_src, d_dst, n, btmin,
-                           e.k64a.p, pos0, e.ends64.p);
-        which = carry_ends ? radix_sort_u64_v64(e.k64a.p, e.ends64.p, e.k64b.p, e.ends64b.p, n, 0,
-                                                bits, tmp, s)
-                           : radix_sort_u64(e.k64a.p, e.v32a.p, e.k64b.p, e.v32b.p, n, 0, bits,
-                                            tmp, s);
+        which = sort_positions(e, d_src, d_dst, d_ts, n, btmin, bits, tmp);
     }
     SortedBatch b;
     b.keys32 = keys32;
@@ -1638,8 +1685,7 @@ void Engine::build(const int32_t* d_src, const int32_t* d_dst, const int64_t* d_
     // the node index is keyed by ids in [0, max_node_id], so a negative id
     // is rejected here, before the store changes
     red64.ensure(minmax_scratch_elems());
-    minmax_ts_min_id(d_ts, d_src, d_dst, n, red64.p, s);
-    check_hip(hipMemcpyAsync(hs, red64.p, 32, hipMemcpyDeviceToHost, s), "read minmax");
+    minmax_ts_min_id(d_ts, d_src, d_dst, n, red64.p, hs, s);  // hs: pinned
     sync();
     if (hs[2] < 0) throw InvalidArgument("node ids must be non-negative");
     // A windowed store settles at about the edges one window of time holds:
@@ -1682,7 +1728,7 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
                         const float* d_feat, size_t n, int64_t tmin, int64_t tmax) {
     hipStream_t s = stream;
     int64_t* hs = reinterpret_cast<int64_t*>(host_scalars);
-    const size_t e_old = E, etot = E + n;
+    const size_t etot = n;  // the store is empty
     // ---- 2. stable radix sort by (ts, position); 32-bit keys when the key
     // range fits (4-byte key traffic per pass instead of 8).  Without edge
     // features the sort's values are the packed endpoints themselves, so the
@@ -1695,14 +1741,11 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
     k64b.ensure(etot);
     ends64.ensure(etot);
     if (carry_ends) ends64b.ensure(etot);
-    v32a.ensure(std::max(etot, 2 * etot));
-    v32b.ensure(std::max(etot, 2 * etot));
     // (sized for the node index's sorts as well, so that it grows once)
     const int id_bits = std::max(1, bit_length_u64(static_cast<uint64_t>(batch_max_id)));
     hist.ensure(radix_tmp_elems(cfg.is_directed ? etot : 2 * etot, id_bits));
     const RadixTmp tmp = radix_tmp(etot, bits);
     uint32_t* k32s[2] = {reinterpret_cast<uint32_t*>(k64a.p), reinterpret_cast<uint32_t*>(k64b.p)};
-    uint32_t* pos0 = carry_ends ? nullptr : v32a.p;
     // the window's cut (step 3), known before the sort: when it keeps every
     // edge and the endpoints ride as values, the sort's last pass writes the
     // new store itself (step 4 then has nothing to do)
@@ -1719,34 +1762,17 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
         ts2.resize(etot);
     }
     const SortedStore st{src2.p, dst2.p, ts2.p, tmin};
-    bool folded = false;
-    int which = 0;
-    if (keys32) {
-        hipLaunchKernelGGL((make_ts_keys_kernel<uint32_t>), dim3(grid_for(etot)), dim3(kB), 0, s,
-                           ts.p, src.p, dst.p, e_old, d_ts, d_src, d_dst, n, tmin, k32s[0], pos0,
-                           ends64.p);
-        if (fold)
-            folded = radix_sort_u32_v64_store(k32s[0], ends64.p, k32s[1], ends64b.p, etot, 0, bits,
-                                              tmp, s, st);
-        else
-            which = carry_ends
-                        ? radix_sort_u32_v64(k32s[0], ends64.p, k32s[1], ends64b.p, etot, 0, bits,
-                                             tmp, s)
-                        : radix_sort_u32(k32s[0], v32a.p, k32s[1], v32b.p, etot, 0, bits, tmp,
-                                         s);
+    int which;
+    if (carry_ends) {
+        const TsSource in{d_ts, d_src, d_dst, tmin};
+        which = keys32 ? radix_sort_ts_u32(in, k32s[0], ends64.p, k32s[1], ends64b.p, etot, bits, tmp, s,
+                                           fold ? &st : nullptr)
+                       : radix_sort_ts_u64(in, k64a.p, ends64.p, k64b.p, ends64b.p, etot, bits, tmp, s,
+                                           fold ? &st : nullptr);
     } else {
-        hipLaunchKernelGGL((make_ts_keys_kernel<uint64_t>), dim3(grid_for(etot)), dim3(kB), 0, s,
-                           ts.p, src.p, dst.p, e_old, d_ts, d_src, d_dst, n, tmin, k64a.p, pos0,
-                           ends64.p);
-        if (fold)
-            folded = radix_sort_u64_v64_store(k64a.p, ends64.p, k64b.p, ends64b.p, etot, 0, bits,
-                                              tmp, s, st);
-        else
-            which = carry_ends
-                        ? radix_sort_u64_v64(k64a.p, ends64.p, k64b.p, ends64b.p, etot, 0, bits,
-                                             tmp, s)
-                        : radix_sort_u64(k64a.p, v32a.p, k64b.p, v32b.p, etot, 0, bits, tmp, s);
+        which = sort_positions(*this, d_src, d_dst, d_ts, etot, tmin, bits, tmp);
     }
+    const bool folded = which < 0;
     uint32_t* perm = which ? v32b.p : v32a.p;
     const uint64_t* sorted_ends = which ? ends64b.p : ends64.p;
 
@@ -1755,11 +1781,10 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
     if (target >= 0) {
         if (keys32)
             hipLaunchKernelGGL((evict_search_kernel<uint32_t>), dim3(1), dim3(1), 0, s,
-                               k32s[which], etot, target, red64.p);
+                               k32s[which], etot, target, hs);
         else
             hipLaunchKernelGGL((evict_search_kernel<uint64_t>), dim3(1), dim3(1), 0, s,
-                               which ? k64b.p : k64a.p, etot, target, red64.p);
-        check_hip(hipMemcpyAsync(hs, red64.p, 24, hipMemcpyDeviceToHost, s), "read evict");
+                               which ? k64b.p : k64a.p, etot, target, hs);
         sync();
         del = static_cast<size_t>(hs[0]);
         store_tmin = static_cast<int64_t>(static_cast<uint64_t>(tmin) + static_cast<uint64_t>(hs[1]));
@@ -1803,12 +1828,12 @@ void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_
             const uint32_t R = 256 / V;
             const size_t blocks = std::min<size_t>((kept + R - 1) / R, 65536);
             hipLaunchKernelGGL(gather_feat_vec_kernel, dim3(blocks ? blocks : 1), dim3(V * R), 0, s,
-                               perm, del, kept, V, reinterpret_cast<const f32x4*>(feat.p), e_old,
+                               perm, del, kept, V, nullptr, size_t{0},
                                reinterpret_cast<const f32x4*>(d_feat),
                                reinterpret_cast<f32x4*>(feat2.p));
         } else {
             hipLaunchKernelGGL(gather_feat_kernel, dim3(grid_capped(kept * feat_dim)), dim3(kB), 0,
-                               s, perm, del, kept, feat_dim, feat.p, e_old, d_feat, feat2.p);
+                               s, perm, del, kept, feat_dim, nullptr, size_t{0}, d_feat, feat2.p);
         }
         feat.swap(feat2);
     }
@@ -1845,11 +1870,10 @@ void Engine::append_store(const int32_t* d_src, const int32_t* d_dst, const int6
     if (cfg.max_time_capacity > 0 && cutoff >= store_tmin) {
         if (keys32)
             hipLaunchKernelGGL((append_evict_kernel<uint32_t>), dim3(1), dim3(1), 0, s, ts.p,
-                               e_old, sk32, n, btmin, cutoff, 1, red64.p);
+                               e_old, sk32, n, btmin, cutoff, 1, hs);
         else
             hipLaunchKernelGGL((append_evict_kernel<uint64_t>), dim3(1), dim3(1), 0, s, ts.p,
-                               e_old, sk64, n, btmin, cutoff, 1, red64.p);
-        check_hip(hipMemcpyAsync(hs, red64.p, 32, hipMemcpyDeviceToHost, s), "read evict");
+                               e_old, sk64, n, btmin, cutoff, 1, hs);
         sync();
         del_old = static_cast<size_t>(hs[0]);
         del_new = static_cast<size_t>(hs[1]);
@@ -1939,11 +1963,10 @@ void Engine::merge_store(const int32_t* d_src, const int32_t* d_dst, const int64
         const int64_t cutoff = latest_ts - cfg.max_time_capacity;
         if (sb.keys32)
             hipLaunchKernelGGL((merge_evict_kernel<uint32_t>), dim3(1), dim3(1), 0, s, ts.p, e_old,
-                               sb.k32, n, btmin, cutoff, red64.p);
+                               sb.k32, n, btmin, cutoff, hs);
         else
             hipLaunchKernelGGL((merge_evict_kernel<uint64_t>), dim3(1), dim3(1), 0, s, ts.p, e_old,
-                               sb.k64, n, btmin, cutoff, red64.p);
-        check_hip(hipMemcpyAsync(hs, red64.p, 32, hipMemcpyDeviceToHost, s), "read evict");
+                               sb.k64, n, btmin, cutoff, hs);
         sync();
         del_old = static_cast<size_t>(hs[0]);
         del_new = static_cast<size_t>(hs[1]);
@@ -2050,13 +2073,12 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
         red32.ensure(4);
         max_i32_pair(src.p, dst.p, E, red32.p, s);
     }
-    flags.ensure(2 * E + 1);
-    scan.ensure(2 * E + 1);
-    scan_scratch.ensure(scan_scratch_elems(2 * E + 1));
-    hipLaunchKernelGGL(ts_group_flags_kernel, dim3(grid_for(E)), dim3(kB), 0, s, ts.p, E, flags.p);
-    exclusive_scan_u32(flags.p, scan.p, E, scan_scratch.p, s);
+    const unsigned spans = static_cast<unsigned>(group_spans(E));
+    gbits.ensure(group_words(cfg.is_directed ? E : 2 * E));
+    gspans.ensure(group_spans(cfg.is_directed ? E : 2 * E));
+    hipLaunchKernelGGL(ts_group_bits_kernel, dim3(spans), dim3(kB), 0, s, ts.p, E, gbits.p, gspans.p);
+    group_scan(gspans.p, spans, reinterpret_cast<uint32_t*>(hs + 1), s);
     if (evicted) check_hip(hipMemcpyAsync(hs, red32.p, 4, hipMemcpyDeviceToHost, s), "read max id");
-    check_hip(hipMemcpyAsync(hs + 1, scan.p + E, 4, hipMemcpyDeviceToHost, s), "read T");
     sync();
     int32_t mx = std::max(max_node_id, batch_max_id);
     uint32_t tg;
@@ -2072,8 +2094,8 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
     tsg_off.resize(T + 1);
     uniq_ts.resize(T);
     erank.resize(E);
-    hipLaunchKernelGGL(ts_group_scatter_kernel, dim3(grid_for(E)), dim3(kB), 0, s, ts.p, E,
-                       flags.p, scan.p, tsg_off.p, uniq_ts.p, time_keys ? 1 : 0, key_t0, erank.p);
+    hipLaunchKernelGGL(ts_group_scatter_kernel, dim3(spans), dim3(kB), 0, s, ts.p, E, gbits.p,
+                       gspans.p, tg, tsg_off.p, uniq_ts.p, time_keys ? 1 : 0, key_t0, erank.p);
     update_neg1_rank(*this);
     check_hip(hipEventRecord(ts_ready, s), "event");
 
@@ -2164,7 +2186,7 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
         // 8-byte ones), else as 64-bit keys of the ids
         flags.ensure(v + 1);
         scan.ensure(v + 1);
-        scan_scratch.ensure(scan_scratch_elems(std::max(v + 1, m2 + 1)));
+        scan_scratch.ensure(scan_scratch_elems(v + 1));
         hipLaunchKernelGGL(active_u32_kernel, dim3(grid_for(v)), dim3(kB), 0, s, active.p, v,
                            flags.p);
         exclusive_scan_u32(flags.p, scan.p, v, scan_scratch.p, s);
@@ -2204,12 +2226,12 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
         // a set at most half full of the distinct pairs
         size_t distinct = m2;
         if (ranked && m2) {
-            flags.ensure(m2 + 1);
-            scan.ensure(m2 + 1);
-            hipLaunchKernelGGL(distinct_flags_kernel, dim3(grid_for(m2)), dim3(kB), 0, s, rkeys, m2,
-                               flags.p);
-            exclusive_scan_u32(flags.p, scan.p, m2, scan_scratch.p, s);
-            check_hip(hipMemcpyAsync(hs, scan.p + m2, 4, hipMemcpyDeviceToHost, s), "read pairs");
+            const unsigned spans2 = static_cast<unsigned>(group_spans(m2));
+            gbits.ensure(group_words(m2));
+            gspans.ensure(spans2);
+            hipLaunchKernelGGL(distinct_bits_kernel, dim3(spans2), dim3(kB), 0, s, rkeys, m2, gbits.p,
+                               gspans.p);
+            group_scan(gspans.p, spans2, reinterpret_cast<uint32_t*>(hs), s);
             sync();
             uint32_t dcount;
             std::memcpy(&dcount, hs, 4);

@@ -242,6 +242,22 @@ struct HostCopy {
 // device (handoff.hip) while the device has engines (attach / detach).
 void attach_lanes(int device);
 void detach_lanes(int device);
+struct HostLane;
+std::vector<std::unique_ptr<HostLane>> take_lanes(int device, int n);
+void give_lanes(int device, std::vector<std::unique_ptr<HostLane>>& lanes);
+constexpr size_t kStageBytes = size_t{8} << 20;  // of a lane's staging buffer
+
+// One lane's pinned buffer for host data on its way to the device through
+// stream s: given back once the stream has read it (done(), or the destructor's
+// wait where a call ends early).
+struct StageLease {
+    int device;
+    hipStream_t s;
+    std::vector<std::unique_ptr<HostLane>> lane;
+    char* take();  // the buffer (kStageBytes)
+    void done();   // the stream has been waited for
+    ~StageLease();
+};
 struct HostLane {
     hipStream_t stream = nullptr;
     void* stage[2] = {nullptr, nullptr};
@@ -345,6 +361,8 @@ struct Engine {
     DBuf<uint64_t> ends64, ends64b;  // packed (src, dst) of the timestamp sort's input
     DBuf<uint32_t> k32a, k32b, v32a, v32b;
     DBuf<uint32_t> hist, flags, scan, scan_scratch;  // hist: radix sort scratch
+    DBuf<uint64_t> gbits;           // group starts (primitives.h): bits,
+    DBuf<uint32_t> gspans, gwords;  // counts per span, groups before every word
     RadixTmp radix_tmp(size_t n, int bits) {
         hist.ensure(radix_tmp_elems(n, bits));
         return RadixTmp{hist.p, hist.cap};
@@ -394,11 +412,8 @@ struct Engine {
     int w_slot_format = 0;  // trw_walk_stats.slot_word_format of the last sample
     int w_replay = 0;
 
-    // pinned host scalars for the few readbacks that size allocations, then
-    // room for a sample's seeds and cutoffs on their way to the device
+    // pinned host scalars for the few readbacks that size allocations
     void* host_scalars = nullptr;
-    static constexpr size_t kScalarBytes = 256;
-    static constexpr size_t kMaxStagedSeeds = 4096;  // 12 bytes each
 
     // a host batch being staged into HBM beside other calls (trw_prefetch_edges):
     // its own device buffers, and the thread that copies

@@ -43,7 +43,7 @@ namespace trw {
 namespace {
 
 constexpr size_t kHuge = size_t(2) << 20;
-constexpr size_t kChunk = size_t(8) << 20;        // bytes of a staging buffer
+constexpr size_t kChunk = kStageBytes;            // bytes of a staging buffer
 constexpr size_t kMinChunk = size_t(512) << 10;   // smallest staged chunk
 constexpr size_t kPackBelow = size_t(2) << 20;    // smaller copies: one kernel
 constexpr int kMaxThreads = 32;
@@ -77,25 +77,8 @@ LanePool& lane_pool() {
 struct Lanes {
     int device;
     std::vector<std::unique_ptr<HostLane>> v;
-    Lanes(int dev, int n) : device(dev) {
-        {
-            LanePool& p = lane_pool();
-            std::lock_guard<std::mutex> g(p.mu);
-            auto& f = p.devices[device].free;
-            while (static_cast<int>(v.size()) < n && !f.empty()) {
-                v.push_back(std::move(f.back()));
-                f.pop_back();
-            }
-        }
-        while (static_cast<int>(v.size()) < n) v.push_back(std::make_unique<HostLane>());
-    }
-    ~Lanes() {
-        LanePool& p = lane_pool();
-        std::lock_guard<std::mutex> g(p.mu);
-        auto& d = p.devices[device];
-        for (auto& l : v)
-            if (d.engines > 0 && d.free.size() < kMaxThreads) d.free.push_back(std::move(l));
-    }
+    Lanes(int dev, int n) : device(dev), v(take_lanes(dev, n)) {}
+    ~Lanes() { give_lanes(device, v); }
 };
 
 // Up to kMaxSegs spans copied by one kernel, 16 bytes per thread: span i is the
@@ -122,6 +105,49 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
 }
 
 }  // namespace
+
+std::vector<std::unique_ptr<HostLane>> take_lanes(int device, int n) {
+    std::vector<std::unique_ptr<HostLane>> v;
+    {
+        LanePool& p = lane_pool();
+        std::lock_guard<std::mutex> g(p.mu);
+        auto& f = p.devices[device].free;
+        while (static_cast<int>(v.size()) < n && !f.empty()) {
+            v.push_back(std::move(f.back()));
+            f.pop_back();
+        }
+    }
+    while (static_cast<int>(v.size()) < n) v.push_back(std::make_unique<HostLane>());
+    return v;
+}
+
+void give_lanes(int device, std::vector<std::unique_ptr<HostLane>>& lanes) {
+    std::vector<std::unique_ptr<HostLane>> rest;  // freed outside the lock
+    LanePool& p = lane_pool();
+    std::lock_guard<std::mutex> g(p.mu);
+    auto& d = p.devices[device];
+    for (auto& l : lanes) {
+        if (d.engines > 0 && d.free.size() < kMaxThreads) d.free.push_back(std::move(l));
+        else rest.push_back(std::move(l));
+    }
+    lanes.clear();
+}
+
+char* StageLease::take() {
+    lane = take_lanes(device, 1);
+    lane[0]->init();
+    return static_cast<char*>(lane[0]->stage[0]);
+}
+
+void StageLease::done() {
+    if (!lane.empty()) give_lanes(device, lane);
+}
+
+StageLease::~StageLease() {
+    if (lane.empty()) return;
+    (void)hipStreamSynchronize(s);
+    give_lanes(device, lane);
+}
 
 void attach_lanes(int device) {
     std::lock_guard<std::mutex> g(lane_pool().mu);

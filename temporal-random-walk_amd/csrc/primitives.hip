@@ -253,7 +253,6 @@ void scan_impl(const T* in, T* out, size_t n, T* scratch, hipStream_t s) {
 // histogram writes and a shorter histogram scan per pass)
 // ---------------------------------------------------------------------------
 constexpr int kMaxDigitBits = 10;
-constexpr int kMaxRadix = 1 << kMaxDigitBits;
 constexpr int kRows = 8;
 constexpr size_t kSortTile = static_cast<size_t>(kBlock) * kRows;
 // The scatter's tile is 8 waves x 4 or 8 rows (sort_plan).
@@ -278,12 +277,23 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid, int db) 
     return m;
 }
 
+// A sort's input already in its buffers.
+template <typename K, typename V>
+struct PtrSource {
+    const K* keys;
+    const V* vals;  // may be null
+    template <typename T>
+    __device__ __forceinline__ T key_as(size_t i) const {
+        return keys[i];
+    }
+    __device__ __forceinline__ V val(size_t i) const { return vals ? vals[i] : V(0); }
+};
+
 // Per-workgroup digit counts of keys[...] >> bit (db-bit digits, the digit
 // masked to dmask), digit-major into hist.  Dynamic
 // LDS: kWaves << db counters.
-template <typename K>
-__global__ __launch_bounds__(kBlock) void radix_upsweep_kernel(const K* __restrict__ keys,
-                                                               size_t n, int bit, int db,
+template <typename K, typename Src>
+__global__ __launch_bounds__(kBlock) void radix_upsweep_kernel(Src in, size_t n, int bit, int db,
                                                                uint32_t dmask, int tiles,
                                                                uint32_t* __restrict__ hist,
                                                                size_t nb) {
@@ -300,7 +310,7 @@ __global__ __launch_bounds__(kBlock) void radix_upsweep_kernel(const K* __restri
 #pragma unroll
         for (int r = 0; r < kRows; ++r) {
             const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
-            key[r] = i < n ? keys[i] : K(0);
+            key[r] = i < n ? in.template key_as<K>(i) : K(0);
         }
         // counts only (no ranks): an LDS atomic per key, which a wave's
         // same-digit lanes serialise among themselves -- the row's lanes with
@@ -395,9 +405,8 @@ struct TileRegs {
     uint32_t rank[Rows];
 };
 
-template <int W, int Rows, typename K, typename V>
-__device__ __forceinline__ void tile_load(const K* __restrict__ keys_in,
-                                          const V* __restrict__ vals_in, size_t n, size_t tile_base,
+template <int W, int Rows, typename K, typename V, typename Src>
+__device__ __forceinline__ void tile_load(const Src& in, size_t n, size_t tile_base,
                                           TileRegs<Rows, K, V>& t) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t wave_base = tile_base + static_cast<size_t>(wave) * Rows * 64;
@@ -405,8 +414,8 @@ __device__ __forceinline__ void tile_load(const K* __restrict__ keys_in,
     for (int r = 0; r < Rows; ++r) {
         const size_t i = wave_base + static_cast<size_t>(r) * 64 + lane;
         const bool valid = i < n;
-        t.key[r] = valid ? keys_in[i] : K(0);
-        t.val[r] = (valid && vals_in) ? vals_in[i] : V(0);
+        t.key[r] = valid ? in.template key_as<K>(i) : K(0);
+        t.val[r] = valid ? in.val(i) : V(0);
     }
 }
 
@@ -484,10 +493,9 @@ __device__ __forceinline__ void tile_write(size_t n, size_t tile_base, int bit, 
 
 // Stable scatter of one digit pass, `tiles` tiles per workgroup.  Dynamic LDS:
 // TileLds::bytes.
-template <typename K, typename V, int Rows, bool Store = false>
+template <typename K, typename V, int Rows, bool Store, typename Src>
 __global__ __launch_bounds__(kScatterBlock) void radix_scatter_kernel(
-    const K* __restrict__ keys_in, const V* __restrict__ vals_in, K* __restrict__ keys_out,
-    V* __restrict__ vals_out, size_t n, int bit, int db, uint32_t dmask, int tiles,
+    Src in, K* __restrict__ keys_out, V* __restrict__ vals_out, size_t n, int bit, int db, uint32_t dmask, int tiles,
     const uint32_t* __restrict__ offsets, size_t nb, const uint32_t* __restrict__ digit_tot,
     SortedStore st = SortedStore{}) {
     extern __shared__ __align__(16) uint32_t s_lds[];
@@ -520,7 +528,7 @@ __global__ __launch_bounds__(kScatterBlock) void radix_scatter_kernel(
         for (int i = threadIdx.x; i < kScatterWaves * R; i += kScatterBlock) l.cnt[i] = 0;
         __syncthreads();
         TileRegs<Rows, K, V> regs;
-        tile_load<kScatterWaves>(keys_in, vals_in, n, tile_base, regs);
+        tile_load<kScatterWaves>(in, n, tile_base, regs);
         tile_rank(n, tile_base, bit, db, dmask, l, regs);
         __syncthreads();
         {
@@ -574,17 +582,17 @@ constexpr int kTileRows = 2;
 constexpr size_t kTileKeys = static_cast<size_t>(kTileBlock) * kTileRows;
 constexpr int kTileDigitBits = 8;
 
-// The keys go round through LDS.  keys_out / vals_out may be the inputs.
-template <typename K, typename V, bool Store = false>
+// The keys go round through LDS.  keys_out / vals_out may be the source's arrays.
+template <typename K, typename V, bool Store, typename Src>
 __global__ __launch_bounds__(kTileBlock) void radix_tile_sort_kernel(
-    const K* keys_in, const V* vals_in, K* keys_out, V* vals_out, uint32_t n, int begin_bit,
-    int end_bit, int db, SortedStore st = SortedStore{}) {
+    Src in, bool with_vals, K* keys_out, V* vals_out, uint32_t n, int begin_bit, int end_bit, int db,
+    SortedStore st = SortedStore{}) {
     extern __shared__ __align__(16) uint32_t s_lds[];
     __shared__ uint32_t s_wave[kTileWaves];
     const int R = 1 << db;
     const TileLds<kTileWaves, kTileRows, K, V> l(s_lds, R);
     TileRegs<kTileRows, K, V> regs;
-    tile_load<kTileWaves>(keys_in, vals_in, n, 0, regs);
+    tile_load<kTileWaves>(in, n, 0, regs);
     for (int i = threadIdx.x; i < R; i += kTileBlock) l.base[i] = 0;
     const int d = threadIdx.x;
     for (int bit = begin_bit; bit < end_bit; bit += db) {
@@ -593,8 +601,7 @@ __global__ __launch_bounds__(kTileBlock) void radix_tile_sort_kernel(
         if (bit != begin_bit) {
             // the keys as the last pass left them (every wave's reads precede
             // the next staging: the barriers below)
-            tile_load<kTileWaves>(static_cast<const K*>(l.key),
-                                   vals_in ? static_cast<const V*>(l.val) : nullptr, n, 0, regs);
+            tile_load<kTileWaves>(PtrSource<K, V>{l.key, with_vals ? l.val : nullptr}, n, 0, regs);
         }
         for (int i = threadIdx.x; i < kTileWaves * R; i += kTileBlock) l.cnt[i] = 0;
         __syncthreads();
@@ -616,7 +623,7 @@ __global__ __launch_bounds__(kTileBlock) void radix_tile_sort_kernel(
             }
         }
         __syncthreads();
-        tile_stage(n, 0, db, vals_in != nullptr, l, regs);
+        tile_stage(n, 0, db, with_vals, l, regs);
         __syncthreads();
     }
     tile_write<Store>(n, 0, 0, 0u, l, keys_out, vals_out, st);  // base[0] = 0: key lp to lp
@@ -666,79 +673,125 @@ SortPlan sort_plan(size_t n, int bits, size_t words) {
     }
 }
 
-// One digit pass's scatter (st: the store to write instead, or nullptr).
-template <int Rows, typename K, typename V>
-void launch_scatter(const SortPlan& p, const K* ki, const V* vi, K* ko, V* vo, size_t n, int bit,
-                    uint32_t dmask, const uint32_t* offsets, const uint32_t* totals,
-                    const SortedStore* st, hipStream_t s) {
+// One digit pass from `in`: histogram, offsets, scatter (st: the store to write
+// instead of ko / vo, or nullptr).
+template <int Rows, typename K, typename V, typename Src>
+void launch_pass(const SortPlan& p, const Src& in, K* ko, V* vo, size_t n, int bit, uint32_t dmask,
+                 uint32_t* hist, const SortedStore* st, hipStream_t s) {
+    const size_t R = size_t{1} << p.db;
+    uint32_t* totals = hist + p.nb * R;
+    const int up_tiles = static_cast<int>(p.tiles * (kScatterBlock * Rows / kSortTile));
+    static_assert(kScatterBlock * kRowsSmall % kSortTile == 0, "whole histogram tiles");
+    hipLaunchKernelGGL((radix_upsweep_kernel<K, Src>), dim3(p.nb), dim3(kBlock),
+                       kWaves * R * sizeof(uint32_t), s, in, n, bit, p.db, dmask, up_tiles, hist,
+                       p.nb);
+    hipLaunchKernelGGL(radix_offsets_kernel, dim3(R), dim3(kBlock), 0, s, hist, p.nb, totals);
     const size_t lds = TileLds<kScatterWaves, Rows, K, V>::bytes(1 << p.db);
     if constexpr (std::is_same<V, uint64_t>::value) {
         if (st) {
-            hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows, true>), dim3(p.nb),
-                               dim3(kScatterBlock), lds, s, ki, vi, nullptr, nullptr, n, bit, p.db,
-                               dmask, p.tiles, offsets, p.nb, totals, *st);
+            hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows, true, Src>), dim3(p.nb),
+                               dim3(kScatterBlock), lds, s, in, nullptr, nullptr, n, bit, p.db, dmask,
+                               p.tiles, hist, p.nb, totals, *st);
             return;
         }
     }
-    hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows>), dim3(p.nb), dim3(kScatterBlock), lds, s,
-                       ki, vi, ko, vo, n, bit, p.db, dmask, p.tiles, offsets, p.nb, totals);
+    hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows, false, Src>), dim3(p.nb),
+                       dim3(kScatterBlock), lds, s, in, ko, vo, n, bit, p.db, dmask, p.tiles, hist,
+                       p.nb, totals);
 }
 
-template <typename K, typename V = uint32_t>
-int radix_sort_impl(K* keys0, V* vals0, K* keys1, V* vals1, size_t n,
+template <typename K, typename V, typename Src>
+__global__ __launch_bounds__(kBlock) void source_copy_kernel(Src in, size_t n, K* __restrict__ keys,
+                                                             V* __restrict__ vals) {
+    const size_t i = blockIdx.x * static_cast<size_t>(kBlock) + threadIdx.x;
+    if (i >= n) return;
+    keys[i] = in.template key_as<K>(i);
+    vals[i] = in.val(i);
+}
+
+// Sorts the n pairs of `in`, which is (keys0, vals0) itself for a PtrSource.
+// Returns which buffer holds the result (-1: the store was written).
+template <typename K, typename V, typename Src>
+int radix_sort_impl(const Src& in, K* keys0, V* vals0, K* keys1, V* vals1, size_t n,
                     int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
                     const SortedStore* store = nullptr) {
-    if (n <= 1 || end_bit <= begin_bit) return 0;
+    constexpr bool in_place = std::is_same<Src, PtrSource<K, V>>::value;
+    if (n <= 1 || end_bit <= begin_bit) {
+        if (!in_place && n) {
+            hipLaunchKernelGGL((source_copy_kernel<K, V, Src>), dim3((n + kBlock - 1) / kBlock),
+                               dim3(kBlock), 0, s, in, n, keys0, vals0);
+            check_hip(hipGetLastError(), "radix sort launch");
+        }
+        return 0;
+    }
     const SortPlan p = sort_plan(n, end_bit - begin_bit, tmp.n);
     if (p.words > tmp.n) throw std::runtime_error("radix sort: scratch too small");
-    const int db = p.db;
-    const size_t R = size_t{1} << db, nb = p.nb;
     K* kb[2] = {keys0, keys1};
     V* vb[2] = {vals0, vals1};
-    constexpr bool can_store = std::is_same<V, uint64_t>::value;
+    const bool with_vals = !in_place || vals0 != nullptr;
     if (p.one_tile) {
-        const size_t lds = TileLds<kTileWaves, kTileRows, K, V>::bytes(static_cast<int>(R));
+        const size_t lds = TileLds<kTileWaves, kTileRows, K, V>::bytes(1 << p.db);
         const int out = p.passes & 1;
         bool stored = false;
-        if constexpr (can_store) {
+        if constexpr (std::is_same<V, uint64_t>::value) {
             if (store) {
-                hipLaunchKernelGGL((radix_tile_sort_kernel<K, V, true>), dim3(1), dim3(kTileBlock),
-                                   lds, s, kb[0], vb[0], nullptr, nullptr,
-                                   static_cast<uint32_t>(n), begin_bit, end_bit, db, *store);
+                hipLaunchKernelGGL((radix_tile_sort_kernel<K, V, true, Src>), dim3(1),
+                                   dim3(kTileBlock), lds, s, in, with_vals, nullptr, nullptr,
+                                   static_cast<uint32_t>(n), begin_bit, end_bit, p.db, *store);
                 stored = true;
             }
         }
         if (!stored)
-            hipLaunchKernelGGL((radix_tile_sort_kernel<K, V>), dim3(1), dim3(kTileBlock), lds, s,
-                               kb[0], vb[0], kb[out], vb[out], static_cast<uint32_t>(n), begin_bit,
-                               end_bit, db);
+            hipLaunchKernelGGL((radix_tile_sort_kernel<K, V, false, Src>), dim3(1),
+                               dim3(kTileBlock), lds, s, in, with_vals, kb[out], vb[out],
+                               static_cast<uint32_t>(n), begin_bit, end_bit, p.db);
         check_hip(hipGetLastError(), "radix sort launch");
-        return out;
+        return stored ? -1 : out;
     }
-    uint32_t* totals = tmp.p + nb * R;
-    const size_t tile = static_cast<size_t>(kScatterBlock) * (p.large ? kRowsLarge : kRowsSmall);
-    const int up_tiles = static_cast<int>(p.tiles * tile / kSortTile);
     int cur = 0;
     for (int pass = 0; pass < p.passes; ++pass) {
-        const int bit = begin_bit + pass * db;
+        const int bit = begin_bit + pass * p.db;
         // the last digit stops at end_bit
-        const int w = end_bit - bit < db ? end_bit - bit : db;
+        const int w = end_bit - bit < p.db ? end_bit - bit : p.db;
         const uint32_t dmask = (1u << w) - 1u;
-        hipLaunchKernelGGL((radix_upsweep_kernel<K>), dim3(nb), dim3(kBlock),
-                           kWaves * R * sizeof(uint32_t), s, kb[cur], n, bit, db, dmask, up_tiles,
-                           tmp.p, nb);
-        hipLaunchKernelGGL(radix_offsets_kernel, dim3(R), dim3(kBlock), 0, s, tmp.p, nb, totals);
         const SortedStore* st = pass == p.passes - 1 ? store : nullptr;
-        if (p.large)
-            launch_scatter<kRowsLarge>(p, kb[cur], vb[cur], kb[cur ^ 1], vb[cur ^ 1], n, bit, dmask,
-                                       tmp.p, totals, st, s);
-        else
-            launch_scatter<kRowsSmall>(p, kb[cur], vb[cur], kb[cur ^ 1], vb[cur ^ 1], n, bit, dmask,
-                                       tmp.p, totals, st, s);
+        auto run = [&](const auto& from) {
+            if (p.large)
+                launch_pass<kRowsLarge>(p, from, kb[cur ^ 1], vb[cur ^ 1], n, bit, dmask, tmp.p, st, s);
+            else
+                launch_pass<kRowsSmall>(p, from, kb[cur ^ 1], vb[cur ^ 1], n, bit, dmask, tmp.p, st, s);
+        };
+        if (pass == 0) run(in);
+        else run(PtrSource<K, V>{kb[cur], vb[cur]});
         check_hip(hipGetLastError(), "radix sort launch");
         cur ^= 1;
     }
-    return cur;
+    return store ? -1 : cur;
+}
+
+// ---------------------------------------------------------------------------
+// group starts: exclusive scan of the spans' counts (one workgroup: 20M
+// positions are 9766 spans)
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(1024) void group_scan_kernel(uint32_t* __restrict__ v, size_t n,
+                                                          uint32_t* __restrict__ total_out) {
+    __shared__ uint32_t s_wave[16];
+    uint32_t carry = 0;
+    for (size_t c = 0; c < n; c += 4096) {
+        const size_t i = c + threadIdx.x * 4u;
+        const u32x4_t x = i < n ? load_u32x4(v, i, n) : u32x4_t{0u, 0u, 0u, 0u};
+        uint32_t tot;
+        uint32_t at = carry + block_exclusive_scan<uint32_t, OpSum, 16>(x.x + x.y + x.z + x.w, &tot,
+                                                                        s_wave);
+        const uint32_t y[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i + k < n) v[i + k] = at;
+            at += y[k];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) *total_out = carry;
 }
 
 // ---------------------------------------------------------------------------
@@ -900,49 +953,43 @@ void running_max_f64(double* data, size_t n, double* scratch, hipStream_t s) {
 
 int radix_sort_u64(uint64_t* keys0, uint32_t* vals0, uint64_t* keys1, uint32_t* vals1, size_t n,
                    int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
-    return radix_sort_impl<uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s);
+    return radix_sort_impl(PtrSource<uint64_t, uint32_t>{keys0, vals0}, keys0, vals0, keys1, vals1, n,
+                           begin_bit, end_bit, tmp, s);
 }
 int radix_sort_u32(uint32_t* keys0, uint32_t* vals0, uint32_t* keys1, uint32_t* vals1, size_t n,
                    int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
-    return radix_sort_impl<uint32_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s);
+    return radix_sort_impl(PtrSource<uint32_t, uint32_t>{keys0, vals0}, keys0, vals0, keys1, vals1, n,
+                           begin_bit, end_bit, tmp, s);
 }
-int radix_sort_u64_v64(uint64_t* keys0, uint64_t* vals0, uint64_t* keys1, uint64_t* vals1,
-                       size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
-    return radix_sort_impl<uint64_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit,
-                                               tmp, s);
+int radix_sort_ts_u32(const TsSource& in, uint32_t* keys0, uint64_t* vals0, uint32_t* keys1,
+                      uint64_t* vals1, size_t n, int bits, RadixTmp tmp, hipStream_t s,
+                      const SortedStore* store) {
+    return radix_sort_impl(in, keys0, vals0, keys1, vals1, n, 0, bits, tmp, s, store);
 }
-int radix_sort_u32_v64(uint32_t* keys0, uint64_t* vals0, uint32_t* keys1, uint64_t* vals1,
-                       size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s) {
-    return radix_sort_impl<uint32_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit,
-                                               tmp, s);
+int radix_sort_ts_u64(const TsSource& in, uint64_t* keys0, uint64_t* vals0, uint64_t* keys1,
+                      uint64_t* vals1, size_t n, int bits, RadixTmp tmp, hipStream_t s,
+                      const SortedStore* store) {
+    return radix_sort_impl(in, keys0, vals0, keys1, vals1, n, 0, bits, tmp, s, store);
+}
+int radix_sort_entries(const EntrySource& in, uint32_t* keys0, uint64_t* vals0, uint32_t* keys1,
+                       uint64_t* vals1, size_t n, int bits, RadixTmp tmp, hipStream_t s) {
+    auto sort = [&](const auto& from) {
+        return radix_sort_impl(from, keys0, vals0, keys1, vals1, n, 0, bits, tmp, s);
+    };
+    if (in.mode == 0) return sort(EntrySourceOf<0>(in));
+    if (in.mode == 1) return sort(EntrySourceOf<1>(in));
+    return sort(EntrySourceOf<2>(in));
+}
+void group_scan(uint32_t* spans, size_t n_spans, uint32_t* host, hipStream_t s) {
+    hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(1024), 0, s, spans, n_spans, host);
+    check_hip(hipGetLastError(), "group scan launch");
 }
 int radix_passes(size_t n, int begin_bit, int end_bit) {
     return n > 1 && end_bit > begin_bit ? sort_plan(n, end_bit - begin_bit, SIZE_MAX).passes : 0;
 }
-bool radix_sort_u32_v64_store(uint32_t* keys0, uint64_t* vals0, uint32_t* keys1, uint64_t* vals1,
-                              size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
-                              const SortedStore& out) {
-    if (n <= 1 || end_bit <= begin_bit) return false;
-    radix_sort_impl<uint32_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s,
-                                        &out);
-    return true;
-}
-bool radix_sort_u64_v64_store(uint64_t* keys0, uint64_t* vals0, uint64_t* keys1, uint64_t* vals1,
-                              size_t n, int begin_bit, int end_bit, RadixTmp tmp, hipStream_t s,
-                              const SortedStore& out) {
-    if (n <= 1 || end_bit <= begin_bit) return false;
-    radix_sort_impl<uint64_t, uint64_t>(keys0, vals0, keys1, vals1, n, begin_bit, end_bit, tmp, s,
-                                        &out);
-    return true;
-}
-
-// Scratch for the reductions lives in a small per-call static device buffer
-// provided by the caller through `out` (2 * kReduceBlocks int64 / doubles
-// beyond out[0..1]).
-void minmax_ts_min_id(const int64_t* v, const int32_t* a, const int32_t* b, size_t n, int64_t* out,
-                      hipStream_t s) {
+void minmax_ts_min_id(const int64_t* v, const int32_t* a, const int32_t* b, size_t n, int64_t* part,
+                      int64_t* out, hipStream_t s) {
     const int nb = reduce_blocks(n);
-    int64_t* part = out + 4;
     hipLaunchKernelGGL(minmax_partial_kernel, dim3(nb), dim3(kBlock), 0, s, v, a, b, n, part);
     hipLaunchKernelGGL(minmax_final_kernel, dim3(1), dim3(kBlock), 0, s, part, nb, out);
     check_hip(hipGetLastError(), "minmax launch");
@@ -957,6 +1004,7 @@ void max_i32_pair(const int32_t* a, const int32_t* b, size_t n, int32_t* out, hi
     check_hip(hipGetLastError(), "max launch");
 }
 
+// Scratch for the sum lives behind out (1024 doubles beyond out[0..1]).
 void sum_f64(const double* v, size_t n, double* out, hipStream_t s) {
     const int nb = reduce_blocks(n);
     double* part = out + 2;

@@ -5,6 +5,7 @@ and the node index stable by (node, position), which numpy's stable argsort
 gives exactly."""
 import numpy as np
 import pytest
+import torch  # noqa: F401  (its HIP runtime comes up before the engine loads the system one)
 
 from temporal_random_walk import capi
 
@@ -40,4 +41,19 @@ def test_store_and_node_index_order_at_the_sort_forms_edges(n, ts_bits, directed
         both = np.stack([s, d], axis=1).ravel()
         out = np.argsort(both, kind="stable") // 2
     np.testing.assert_array_equal(eng.array("node_ts_sorted_outbound_indices"), out)
+    # the groups: runs of equal timestamps in the store, and of equal (node,
+    # timestamp) in the node index
+    t = ts[order]
+    np.testing.assert_array_equal(eng.array("timestamp_group_offsets"), _starts(t[1:] != t[:-1], n))
+    node = s[out] if directed else np.sort(both, kind="stable")
+    starts = _starts((node[1:] != node[:-1]) | (t[out][1:] != t[out][:-1]), out.size)
+    np.testing.assert_array_equal(eng.array("node_ts_group_outbound_offsets"), starts[:-1])
+    first = np.searchsorted(node, np.arange(int(max(s.max(), d.max())) + 2))
+    np.testing.assert_array_equal(eng.array("count_ts_group_per_node_outbound"),
+                                  np.searchsorted(starts[:-1], first))
     eng.close()
+
+
+def _starts(changes, n):
+    """Positions starting a run (changes: where position i + 1 differs from i), then n."""
+    return np.concatenate([[0], np.nonzero(changes)[0] + 1, [n]]).astype(np.uint64)

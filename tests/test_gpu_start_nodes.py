@@ -3,6 +3,7 @@ wpn walks each, at the edges of the id blocks, through the flags (ids no more
 than the batch's entries) and through the sort (sparse ids)."""
 import numpy as np
 import pytest
+import torch  # noqa: F401  (its HIP runtime comes up before the engine loads the system one)
 
 from temporal_random_walk import capi
 

@@ -3,6 +3,7 @@ walk's length, for dims on both sides of the 16-byte path and slot counts that
 end inside a workgroup's run."""
 import numpy as np
 import pytest
+import torch  # noqa: F401  (its HIP runtime comes up before the engine loads the system one)
 
 from temporal_random_walk import capi
 from tests import graphs
