@@ -80,21 +80,57 @@ __device__ __forceinline__ T block_sum(T v, T* s_wave) {
 
 // ---------------------------------------------------------------------------
 // scan: tile = 256 threads x 16 consecutive items per thread
+//
+// A thread owns 16 consecutive items, so that sums are rounded in one order
+// whatever the launch; read that way a wave's access touches 64 lines of 128
+// bytes for 512 bytes of doubles.  The tile therefore passes through LDS: memory
+// is read and written in rows of 256 consecutive items, a thread's run is padded
+// by one item (17 doubles apart, lanes hit distinct banks).  Same sums, bit for
+// bit; bound by HBM.
 // ---------------------------------------------------------------------------
 constexpr int kScanItems = 16;
 constexpr size_t kScanTile = static_cast<size_t>(kBlock) * kScanItems;
+constexpr size_t kScanLds = kScanTile + kBlock;
+
+// This thread's items of the tile at t0 (pad past n), through lds (kScanLds).
+template <typename T>
+__device__ __forceinline__ void scan_tile_load(const T* in, size_t t0, size_t n, T pad, T* lds,
+                                               T (&v)[kScanItems]) {
+#pragma unroll
+    for (int r = 0; r < kScanItems; ++r) {
+        const uint32_t i = r * kBlock + threadIdx.x;
+        lds[i + i / kScanItems] = t0 + i < n ? in[t0 + i] : pad;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j) v[j] = lds[threadIdx.x * (kScanItems + 1) + j];
+}
+
+// Writes the tile at t0 from the threads' items; lds was last read by
+// scan_tile_load (a thread overwrites only what it has read itself).
+template <typename T>
+__device__ __forceinline__ void scan_tile_store(T* out, size_t t0, size_t n, T* lds,
+                                                const T (&v)[kScanItems]) {
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j) lds[threadIdx.x * (kScanItems + 1) + j] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kScanItems; ++r) {
+        const uint32_t i = r * kBlock + threadIdx.x;
+        if (t0 + i < n) out[t0 + i] = lds[i + i / kScanItems];
+    }
+}
 
 template <typename T, typename Op>
 __global__ __launch_bounds__(kBlock) void scan_reduce_kernel(const T* __restrict__ in, size_t n,
                                                              T* __restrict__ sums) {
     __shared__ T s_wave[kWaves];
-    const size_t base = blockIdx.x * kScanTile + static_cast<size_t>(threadIdx.x) * kScanItems;
+    __shared__ T s_tile[kScanLds];
+    T v[kScanItems];
+    scan_tile_load(in, blockIdx.x * kScanTile, n, Op::template identity<T>(), s_tile, v);
     T acc = Op::template identity<T>();
 #pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        const size_t i = base + j;
-        if (i < n) acc = Op::apply(acc, in[i]);
-    }
+    for (int j = 0; j < kScanItems; ++j) acc = Op::apply(acc, v[j]);
     const T tot = block_sum<T, Op>(acc, s_wave);
     if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
@@ -132,24 +168,23 @@ template <typename T, bool Inclusive, typename Op>
 __global__ __launch_bounds__(kBlock) void scan_apply_kernel(const T* in, T* out, size_t n,
                                                             const T* __restrict__ sums) {
     __shared__ T s_wave[kWaves];
-    const size_t base = blockIdx.x * kScanTile + static_cast<size_t>(threadIdx.x) * kScanItems;
+    __shared__ T s_tile[kScanLds];
+    const size_t t0 = blockIdx.x * kScanTile;
     T v[kScanItems];
+    scan_tile_load(in, t0, n, Op::template identity<T>(), s_tile, v);
     T acc = Op::template identity<T>();
 #pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        const size_t i = base + j;
-        v[j] = i < n ? in[i] : Op::template identity<T>();
-        acc = Op::apply(acc, v[j]);
-    }
+    for (int j = 0; j < kScanItems; ++j) acc = Op::apply(acc, v[j]);
     T tot;
     T run = Op::apply(sums[blockIdx.x], block_exclusive_scan<T, Op>(acc, &tot, s_wave));
 #pragma unroll
     for (int j = 0; j < kScanItems; ++j) {
-        const size_t i = base + j;
-        if (Inclusive) run = Op::apply(run, v[j]);
-        if (i < n) out[i] = run;
-        if (!Inclusive) run = Op::apply(run, v[j]);
+        const T x = v[j];
+        if (Inclusive) run = Op::apply(run, x);
+        v[j] = run;
+        if (!Inclusive) run = Op::apply(run, x);
     }
+    scan_tile_store(out, t0, n, s_tile, v);
     if (!Inclusive && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = sums[gridDim.x];
 }
 
