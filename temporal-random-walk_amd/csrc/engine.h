@@ -159,7 +159,7 @@ struct SampleSpace {
         used = off + n * sizeof(T);
         return reinterpret_cast<T*>(base + off);
     }
-    // scratch of a radix sort of n keys of `bits` bits
+    // scratch of radix sorts of up to n keys of `bits` bits
     RadixTmp sort_tmp(DBuf<uint32_t>& own, size_t n, int bits) {
         const size_t want = radix_tmp_elems(n, bits);
         if (base && want <= sort_words) return RadixTmp{sort, sort_words};

@@ -44,8 +44,9 @@ void running_max_f64(double* data, size_t n, double* scratch, hipStream_t s);
 // Stable sort of (key, value) pairs by key bits [begin_bit, end_bit).  Values
 // may be null (keys only).  Buffers are ping-ponged; the function returns 0 if
 // the sorted result ended in (keys0, vals0) and 1 if in (keys1, vals1).
-// tmp: device scratch; radix_tmp_elems(n, end_bit - begin_bit) words let every
-// size run its fastest form, radix_min_elems words let it run.
+// tmp: device scratch; radix_tmp_elems(n, end_bit - begin_bit) words let a sort
+// of n keys, or of any fewer, run its fastest form, radix_min_elems words let it
+// run.
 struct RadixTmp {
     uint32_t* p;
     size_t n;  // words

@@ -954,12 +954,20 @@ int reduce_blocks(size_t n) {
 }  // namespace
 
 size_t scan_scratch_elems(size_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
-size_t radix_tmp_elems(size_t n, int bits) {
-    return n <= 1 || bits <= 0 ? 1 : std::max<size_t>(sort_plan(n, bits, SIZE_MAX).words, 1);
+// A sort's need does not grow with n throughout: it falls where digits become
+// narrower (past kWideMax), where workgroups take two tiles (past kSortBlocks
+// of them) and where tiles become larger (from kLargeMin on).  The scratch of n
+// keys is therefore the largest of n's own and of the need just below each of
+// those sizes.
+static size_t scratch_words(size_t n, int bits, size_t words) {
+    if (n <= 1 || bits <= 0) return 1;
+    size_t most = 1;
+    for (const size_t m : {n, kWideMax, kSortBlocks * kScatterBlock * kRowsSmall, kLargeMin - 1})
+        if (m <= n) most = std::max(most, sort_plan(m, bits, words).words);
+    return most;
 }
-size_t radix_min_elems(size_t n, int bits) {
-    return n <= 1 || bits <= 0 ? 1 : std::max<size_t>(sort_plan(n, bits, 0).words, 1);
-}
+size_t radix_tmp_elems(size_t n, int bits) { return scratch_words(n, bits, SIZE_MAX); }
+size_t radix_min_elems(size_t n, int bits) { return scratch_words(n, bits, 0); }
 
 void exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* scratch,
                         hipStream_t s) {

@@ -2485,7 +2485,7 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
         uint32_t* kb[2] = {sp.take(ng_keys0, nw), sp.take(ng_keys1, nw)};
         uint32_t* vb[2] = {sp.take(ng_vals0, nw), sp.take(ng_vals1, nw)};
         const int nbits = std::max(1, bit_length(static_cast<uint64_t>(std::max(max_node_id, 0))));
-        const RadixTmp hi = sp.sort_tmp(hist, nw, nbits);
+        const RadixTmp hi = sp.sort_tmp(hist, nw, nbits);  // of every regrouping: live <= nw
         uint32_t* cnt = sp.take(ng_count, 1);
         check_hip(hipMemsetAsync(cnt, 0, 4, s), "live count clear");
         int in = 0;  // the pair the next list is emitted into
