@@ -361,8 +361,8 @@ trw_status trw_get_walk_stats(void* handle, trw_walk_stats* out);
 
 /* ---- test hooks ---------------------------------------------------------- */
 
-/* After this call, the next n device allocations of any handle succeed and the
- * one after them fails as out of memory (TRW_ERR_OUT_OF_MEMORY), its retry
+/* After this call, the next n allocations of any handle (device memory, or a
+ * host copy's pinned staging) succeed and the one after them fails as out of memory (TRW_ERR_OUT_OF_MEMORY), its retry
  * included; n < 0 disarms.  For tests of the failure paths: an ingest that
  * fails after its batch was accepted leaves the handle empty, as after
  * trw_clear.  No counterpart in the reference. */

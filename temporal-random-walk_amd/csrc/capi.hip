@@ -23,7 +23,8 @@ Engine::Engine(const trw_config& c) : cfg(c), device(c.device_id) {
     check_hip(hipEventCreateWithFlags(&side_done, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventCreateWithFlags(&ts_ready, hipEventDisableTiming), "hipEventCreate");
     for (auto& e : ev) check_hip(hipEventCreate(&e), "hipEventCreate");
-    check_hip(hipHostMalloc(&host_scalars, 256, hipHostMallocDefault), "hipHostMalloc");
+    check_hip(hipHostMalloc(&host_scalars, kHostScalarBytes + kSeedStageBytes, hipHostMallocDefault),
+              "hipHostMalloc");
     attach_lanes(device);
 }
 

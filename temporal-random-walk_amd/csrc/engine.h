@@ -32,6 +32,8 @@ struct InvalidArgument : std::invalid_argument {
 // its retry fails too), or only at its first attempt
 // (trw_debug_fail_allocation_transient: the retry after releasing the retired
 // blocks succeeds).
+// A lane taken from the handoff's pool counts as an allocation for the first:
+// the pool makes one where it has none free.
 inline std::atomic<long long> g_alloc_fail_after{-1};
 inline std::atomic<long long> g_alloc_fail_transient{-1};
 inline bool alloc_hook_fires(std::atomic<long long>& c) {
@@ -246,6 +248,10 @@ struct HostLane;
 std::vector<std::unique_ptr<HostLane>> take_lanes(int device, int n);
 void give_lanes(int device, std::vector<std::unique_ptr<HostLane>>& lanes);
 constexpr size_t kStageBytes = size_t{8} << 20;  // of a lane's staging buffer
+// A handle's own pinned block: scalars read back, then seeds (and cutoffs) on
+// their way to the device.
+constexpr size_t kHostScalarBytes = 256;
+constexpr size_t kSeedStageBytes = size_t{256} << 10;
 
 // One lane's pinned buffer for host data on its way to the device through
 // stream s: given back once the stream has read it (done(), or the destructor's
@@ -412,7 +418,8 @@ struct Engine {
     int w_slot_format = 0;  // trw_walk_stats.slot_word_format of the last sample
     int w_replay = 0;
 
-    // pinned host scalars for the few readbacks that size allocations
+    // pinned host scalars for the few readbacks that size allocations (and the
+    // seeds' staging behind them)
     void* host_scalars = nullptr;
 
     // a host batch being staged into HBM beside other calls (trw_prefetch_edges):

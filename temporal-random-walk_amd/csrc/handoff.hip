@@ -107,6 +107,7 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
 }  // namespace
 
 std::vector<std::unique_ptr<HostLane>> take_lanes(int device, int n) {
+    if (alloc_hook_fires(g_alloc_fail_after)) throw std::bad_alloc();
     std::vector<std::unique_ptr<HostLane>> v;
     {
         LanePool& p = lane_pool();

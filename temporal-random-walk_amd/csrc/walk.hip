@@ -2061,7 +2061,7 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
     bool have_starts = false, have_cutoffs = false;
     int32_t* a_starts = nullptr;
     int64_t* a_cutoffs = nullptr;
-    StageLease lease{device, s, {}};      // seeds on their way to the device
+    StageLease lease{device, s, {}};      // many seeds on their way to the device
     const int32_t* start_ids = nullptr;   // the start nodes, wpn walks each
     const int64_t* start_cuts = nullptr;  // and their cutoffs
     auto bit_length = [](uint64_t v) { return v ? 64 - __builtin_clzll(v) : 0; };
@@ -2159,17 +2159,21 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
             nw = static_cast<uint64_t>(ns) * static_cast<uint64_t>(wpn);
             if (into && nw > into->capacity_walks)
                 throw InvalidArgument("the sample has more walks than the outputs' capacity");
-            // cutoffs (when given), then seeds, in one buffer: through a
-            // pinned buffer in one copy that the call's end waits for, or --
-            // past its size -- copied from the caller's arrays
+            // cutoffs (when given), then seeds, in one buffer: in one copy
+            // through the handle's pinned block or -- past its size, where
+            // the call may allocate -- a lane's, which the call's end waits
+            // for; else copied from the caller's arrays
             const size_t nc = p.cutoff_times ? ns : 0;
             int64_t* buf = sp.take(s_seeds, nc + (ns + 1) / 2);
             int32_t* seeds = reinterpret_cast<int32_t*>(buf + nc);
-            if (ns && nc * 8 + ns * 4 <= kStageBytes) {
-                char* stage = lease.take();
+            const size_t bytes = nc * 8 + ns * 4;
+            char* stage = nullptr;
+            if (bytes <= kSeedStageBytes) stage = static_cast<char*>(host_scalars) + kHostScalarBytes;
+            else if (!into && bytes <= kStageBytes) stage = lease.take();
+            if (ns && stage) {
                 if (nc) std::memcpy(stage, p.cutoff_times, nc * 8);
                 std::memcpy(stage + nc * 8, p.seed_nodes, ns * 4);
-                check_hip(hipMemcpyAsync(buf, stage, nc * 8 + ns * 4, hipMemcpyHostToDevice, s),
+                check_hip(hipMemcpyAsync(buf, stage, bytes, hipMemcpyHostToDevice, s),
                           "seeds H2D");
             } else if (ns) {
                 check_hip(hipMemcpyAsync(seeds, p.seed_nodes, ns * 4, hipMemcpyHostToDevice, s),

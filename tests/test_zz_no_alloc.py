@@ -173,6 +173,28 @@ def test_noalloc_sample_weight_pickers():
     eng.close()
 
 
+# 12 bytes a seed with its cutoff, 4 without: at both sides of the handle's
+# 256 KiB staging block
+@pytest.mark.parametrize("n,cutoffs", [(1, True), (21_845, True), (21_846, True),
+                                       (65_536, False), (65_537, False)])
+def test_noalloc_seeds_of_a_handle_fed_on_the_device(n, cutoffs):
+    """No pinned staging is made or taken for the seeds (the armed hook counts a
+    lane of the host copies as an allocation), also on a handle that has made
+    no host copy yet."""
+    import torch
+    from temporal_random_walk import capi
+    s, d, t = graphs.powerlaw(20_000, 300_000, n_ts=5_000, seed=5)
+    dv = [torch.from_numpy(x).cuda() for x in (s, d, t)]
+    torch.cuda.synchronize()
+    eng = capi.Engine(is_directed=True, global_seed=9, shuffle_walk_order=True)
+    eng.add_edges_device(dv[0].data_ptr(), dv[1].data_ptr(), dv[2].data_ptr(), len(s), None, 0)
+    rng = np.random.default_rng(n)
+    seeds = rng.choice(s, n).astype(np.int32)
+    cut = rng.integers(0, t.max() + 2, n).astype(np.int64) if cutoffs else None
+    assert _same(eng, n + 5, 12, 0, "nodes", "Linear", 1, seed_nodes=seeds, cutoff_times=cut) == n
+    eng.close()
+
+
 def test_noalloc_calls_of_two_handles_from_two_threads():
     """Two handles on one device, each sampling from its own thread: the
     device's scratch array is taken in turn, so both threads' walks equal
