@@ -1590,6 +1590,20 @@ static_assert(kLayoutWalks == kScratchTile, "a layout workgroup owns one scratch
 // measured 1.3 ms slower over 10M walks than in one.
 constexpr int kLayoutPackedMaxSlots = 120;
 
+// Edge features: 16-byte loads a thread has in flight, and the dimensions
+// (multiples of this many floats, 64 bytes) whose rows the layout pass writes from the
+// edge ids it holds, instead of gather_walk_features_kernel from the laid-out
+// ones.  The pass saves reading those (8 bytes a slot) and takes the features of
+// walks that start close in time together, but writes walk by walk, and walks
+// that do not end on 64 bytes leave partial blocks.  3.75M backward walks of 40,
+// sampling call, gather and layout pass, means over where the buffers lay (each
+// moves by up to 10 %): dim 4 5.07 and 5.09 ms, dim 8 5.44 and 5.47 (0.15M walks
+// of 100: 0.50 and 0.52), dim 20 7.09 and 7.17; dim 16 6.34 and 6.13,
+// dim 32 8.34 and 8.09; 0.9M walks, dim 48 2.72 and 2.62, dim 64 3.17
+// and 2.83 (one load in flight 2.99).
+constexpr int kFeatUnits = 4;
+constexpr size_t kFeatLayoutDims = 16;
+
 struct LayoutArgs {
     const uint64_t* sp;  // scratch slot words
     int pk_nb, pk_rb;    // their node and rank field widths
@@ -1604,6 +1618,11 @@ struct LayoutArgs {
     KeyTimes kt;
     const uint32_t* order;  // walk of each scratch column (nullptr: the column index)
     uint64_t q0, q_end;     // scratch columns [q0, q_end) of this launch (q0 % 64 == 0)
+    // edge features of the edge-id slots (fv = feature_dim / 4 vectors per
+    // slot; 0: written by gather_walk_features_kernel)
+    const float* feat;
+    float* of;
+    uint32_t fv;
 };
 
 // Value of output slot i of a row whose first `cw` slots were written (v: the
@@ -1663,6 +1682,39 @@ __device__ __forceinline__ void layout_rows(const LayoutArgs& a, const int* cnt,
             if (Arr == 0) __builtin_nontemporal_store(static_cast<int32_t>(y), a.on + base + i);
             else if (Arr == 1) __builtin_nontemporal_store(y, a.ot + base + i);
             else __builtin_nontemporal_store(y, a.oe + base + i);
+        }
+    }
+    if (Arr != 2 || !a.fv) return;
+    for (int wl2 = wave; wl2 < kLayoutWalks; wl2 += 4) {
+        if (w0 + wl2 >= a.q_end) break;
+        const uint64_t base = static_cast<uint64_t>(row[wl2]) * static_cast<uint64_t>(K) + k0;
+        const int n = cnt[wl2];
+        const int cw = n - 1 - k0;
+        // the slots' edge features (finalize_host_walks,
+        // walks_with_edge_features_host.cuh:44-62), from the edge ids in
+        // the tile: row [slot][dim] of the walk, zeros past the count
+        const uint32_t fv = a.fv;
+        const f32x4* feat = reinterpret_cast<const f32x4*>(a.feat);
+        f32x4* of = reinterpret_cast<f32x4*>(a.of) + base * fv;
+        const uint32_t units = static_cast<uint32_t>(kc) * fv;
+        for (uint32_t t0 = lane; t0 < units; t0 += 64 * kFeatUnits) {
+            f32x4 v[kFeatUnits];
+#pragma unroll
+            for (int k = 0; k < kFeatUnits; ++k) {
+                const uint32_t t = t0 + 64u * k;
+                const int i = static_cast<int>(t / fv);
+                const uint32_t c = t - static_cast<uint32_t>(i) * fv;
+                v[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (t < units && i < cw) {
+                    const uint64_t e = static_cast<uint64_t>(word_eid(word_at(wl2, n, cw, i), a.pk_nb, a.pk_rb));
+                    v[k] = feat[e * fv + c];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kFeatUnits; ++k) {
+                const uint32_t t = t0 + 64u * k;
+                if (t < units) __builtin_nontemporal_store(v[k], of + t);
+            }
         }
     }
 }
@@ -1885,12 +1937,8 @@ __global__ void u32_from_i32_kernel(const int32_t* __restrict__ a, uint64_t n,
 // units of one T (16 bytes where dim is a multiple of 4), kFeatUnits per
 // thread at a time so that many row loads are in flight.  Bound by the output's
 // writes and the row reads: 1M forward walks of 25 with dim 8 (768 MB written)
-// 168 us, against 580 us with one value and a 64-bit division per thread; 3.75M
-// backward walks of 40 with dim 16 (9.4 GB) 2.41 ms, 3.9 TB/s written.  (The
-// layout pass writing the features of its own rows took 4.01 ms, without them
-// 1.34 ms.)
+// 168 us, against 580 us with one value and a 64-bit division per thread.
 constexpr uint32_t kFeatSlots = 1024;
-constexpr int kFeatUnits = 4;
 template <typename T>
 __global__ __launch_bounds__(kB) void gather_walk_features_kernel(
     const int64_t* __restrict__ eids, uint64_t slots, uint32_t per, uint32_t units,
@@ -2532,6 +2580,9 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
 #undef TRW_LAUNCH
 #undef TRW_LAUNCH_FAMILY
     check_hip(hipEventRecord(ev[6], s), "event");
+    // (a row chunk's 16-byte units number below 2^31)
+    const bool feat_in_layout = eslots && !rows_direct && feat_dim > 0 &&
+                                feat_dim % kFeatLayoutDims == 0 && feat_dim < (size_t{1} << 24);
     if (nw && L > 0 && !rows_direct) {
         LayoutArgs la{};
         la.sp = a.packed;
@@ -2550,6 +2601,13 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
         la.order = a.order;
         la.q0 = 0;
         la.q_end = nw;
+        // (device buffers are 256-byte aligned, the caller's 16-byte aligned)
+        if (feat_in_layout) {
+            if (!into) w_feat.resize(eslots * feat_dim);
+            la.feat = feat.p;
+            la.of = into ? into->feat : w_feat.p;
+            la.fv = static_cast<uint32_t>(feat_dim / 4);
+        }
         const size_t tile = static_cast<size_t>(la.C + 1) * (kLayoutWalks + 1) * sizeof(uint64_t);
         const size_t lds = tile + kLayoutWalks * (sizeof(int) + sizeof(uint32_t));
         const unsigned gx = static_cast<unsigned>((nw + kLayoutWalks - 1) / kLayoutWalks);
@@ -2558,9 +2616,11 @@ void Engine::sample(const trw_sample_params& p, const SampleTarget* into) {
     }
 
     // ---- edge features of every walk slot (finalize_host_walks,
-    // walks_with_edge_features_host.cuh:44-62, on device), from the laid-out
-    // edge ids
-    if (feat_dim > 0 && eslots) {
+    // walks_with_edge_features_host.cuh:44-62, on device) that the layout pass
+    // has not written, from the laid-out edge ids
+    if (feat_in_layout) {
+        // written
+    } else if (feat_dim > 0 && eslots) {
         if (!into) w_feat.resize(eslots * feat_dim);
         float* of = into ? into->feat : w_feat.p;
         const uint32_t dim = static_cast<uint32_t>(feat_dim);

@@ -102,7 +102,7 @@ def _same(eng, cap, L, dim, mode, bias, n, **kw):
     return nw
 
 
-@pytest.mark.parametrize("dim", [8, 6])
+@pytest.mark.parametrize("dim", [16, 8, 6])
 def test_noalloc_sample_equals_sample_device(dim):
     eng = _engine(dim)
     cap = 100_000
