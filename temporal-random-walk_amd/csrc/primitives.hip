@@ -425,7 +425,7 @@ struct TileLds {
         key = reinterpret_cast<K*>(base + R);
         val = reinterpret_cast<V*>(key + kTile);
     }
-    static size_t bytes(int R) {
+    static constexpr size_t bytes(int R) {
         return (static_cast<size_t>(W) + 2) * R * sizeof(uint32_t) + kTile * (sizeof(K) + sizeof(V));
     }
 };
@@ -682,6 +682,7 @@ constexpr size_t kWideMax = size_t{1} << 19;
 constexpr size_t kLargeMin = size_t{3} << 22;
 constexpr int kDigitBits = 8;
 constexpr size_t kSortBlocks = 1024;
+constexpr size_t kLdsBytes = size_t{160} << 10;  // of a CU, and the most a workgroup may take
 
 struct SortPlan {
     bool one_tile, large;
@@ -721,7 +722,12 @@ void launch_pass(const SortPlan& p, const Src& in, K* ko, V* vo, size_t n, int b
                        kWaves * R * sizeof(uint32_t), s, in, n, bit, p.db, dmask, up_tiles, hist,
                        p.nb);
     hipLaunchKernelGGL(radix_offsets_kernel, dim3(R), dim3(kBlock), 0, s, hist, p.nb, totals);
-    const size_t lds = TileLds<kScatterWaves, Rows, K, V>::bytes(1 << p.db);
+    using Lds = TileLds<kScatterWaves, Rows, K, V>;
+    // 64-bit keys and values take 72 KiB at 10-bit digits, 74 KiB with large tiles
+    // at 8: two such workgroups fit a CU
+    static_assert(Lds::bytes(1 << (Rows == kRowsLarge ? kDigitBits : kMaxDigitBits)) <= kLdsBytes / 2,
+                  "two workgroups per CU");
+    const size_t lds = Lds::bytes(1 << p.db);
     if constexpr (std::is_same<V, uint64_t>::value) {
         if (st) {
             hipLaunchKernelGGL((radix_scatter_kernel<K, V, Rows, true, Src>), dim3(p.nb),

@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
     (1, 8), (2, 1), (64, 33), (1023, 20), (2047, 8), (2048, 9), (2049, 9), (4097, 33),
     (100_001, 20), (262_145, 27), (524_288, 20), (524_289, 20), (2_097_153, 30),
     (6_291_456, 17), (12_582_912, 12),
+    (100_001, 40), (12_582_912, 40),  # the widest LDS tiles: 72 and 74 KiB
 ])
 def test_store_and_node_index_order_at_the_sort_forms_edges(n, ts_bits, directed):
     if n > 6_291_456 and not directed:
