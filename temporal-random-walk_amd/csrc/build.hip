@@ -1734,13 +1734,11 @@ void Engine::build(const int32_t* d_src, const int32_t* d_dst, const int64_t* d_
     }
 }
 
-// Steps 2-4 of an ingest, general case: one stable LSD radix sort of
-// (ts - tmin, position) over the old store followed by the batch -- identical
-// to the reference's "sort the batch, stable-merge it after the old store"
-// (temporal_graph.cu:67-134) because the old store is already sorted and
-// precedes the batch -- then the window eviction as an upper_bound on the
-// sorted keys (temporal_graph.cu:136-156) and the gather of the kept suffix.
-// tmin / tmax span the store and the batch.
+// Steps 2-4 of an ingest into an empty store: one stable LSD radix sort of the
+// batch by (ts - tmin, position) -- the reference's "sort the batch" (its merge
+// into the store, temporal_graph.cu:67-134, has nothing to merge with) -- then the
+// window eviction as an upper_bound on the sorted keys (temporal_graph.cu:136-156)
+// and the gather of the kept suffix.  tmin / tmax span the batch.
 void Engine::sort_store(const int32_t* d_src, const int32_t* d_dst, const int64_t* d_ts,
                         const float* d_feat, size_t n, int64_t tmin, int64_t tmax) {
     hipStream_t s = stream;

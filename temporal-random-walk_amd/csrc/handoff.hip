@@ -18,8 +18,9 @@
 //    kernel on the engine's stream that moves every array (a runtime copy of
 //    pageable memory costs some 10 us per array): walks from 32 seeds 156 ->
 //    120 us.
-// Lanes are kept for the process in a pool per device: pinning their 16 MiB
-// takes longer than most copies, and a new handle need not pay it again.
+// Lanes are kept in a pool per device, shared by its handles, until the last of
+// them ends: pinning their 16 MiB takes longer than most copies, and a handle
+// beside others need not pay it again.
 // Host-pointer ingest (trw_add_edges) uses the same lanes in the other
 // direction: the reference copies each batch array with one blocking
 // cudaMemcpy (data/buffer.cuh:135-149).
