@@ -2103,7 +2103,12 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
     T = tg;
     const uint64_t range =
         T ? static_cast<uint64_t>(store_tmax) - static_cast<uint64_t>(store_tmin) : 0;
-    time_keys = T > 0 && range <= kTimeKeyMax && range + 1 <= kTimeKeyGap * T;
+    // bits a slot word has for a time (sample() lays the words out)
+    const int slot_bits = 64 - std::max(1, bit_length_u64(static_cast<uint64_t>(std::max(max_node_id, 0)))) -
+                          bit_length_u64(E ? E - 1 : 0);
+    const bool weights = cfg.enable_weight_computation || cfg.enable_temporal_node2vec;
+    time_keys = T > 0 && range <= kTimeKeyMax && range + 1 <= kTimeKeyGap * T &&
+                (range + 1 == T || T > kRankTableMax || weights || bit_length_u64(T) > slot_bits);
     key_t0 = store_tmin;
     key_max = time_keys ? range : (T ? T - 1 : 0);
     tsg_off.resize(T + 1);
@@ -2116,8 +2121,6 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
 
     // ---- 5a. the key blocks of slot words that cannot hold a whole key, on
     // the side stream (read by the walks only)
-    const int slot_bits = 64 - std::max(1, bit_length_u64(static_cast<uint64_t>(std::max(max_node_id, 0)))) -
-                          bit_length_u64(E ? E - 1 : 0);
     const bool key_blocks = time_keys && slot_bits > 0 && slot_bits < bit_length_u64(key_max + 1);
     kblk_shift = -1;
     if (key_blocks) {
@@ -2133,7 +2136,6 @@ void Engine::build_accepted(const int32_t* d_src, const int32_t* d_dst, const in
     // stream, beside the node index: they read only the timestamp groups.
     // Pivots are the store's min/max ts.  Their buffers are the side's own.
     weights_ready = false;
-    const bool weights = cfg.enable_weight_computation || cfg.enable_temporal_node2vec;
     if (weights) {
         hipStream_t sd = side;
         check_hip(hipStreamWaitEvent(sd, ts_ready, 0), "wait timestamp groups");

@@ -72,13 +72,26 @@ namespace trw {
 // ---- time keys --------------------------------------------------------------
 // The index and the walks order times by a 32-bit key.  "Rank" in a name or a
 // comment here means this key.  It is the timestamp's rank among the graph's
-// unique timestamps, or -- where most time units of the store's span occur
-// (span + 1 <= kTimeKeyGap * unique timestamps) -- its offset from the store's
-// first timestamp.  Both order exactly as the timestamps do; the offset turns
-// back into the timestamp by an addition, the rank by a lookup in uniq_ts.
-// Gapped graphs keep ranks: their hubs then have a group at (nearly) every
-// key of their span, which the bucket tables answer without a search.
+// unique timestamps, or its offset from the store's first timestamp.  Both order
+// exactly as the timestamps do; the offset turns back into the timestamp by an
+// addition, the rank by a lookup in uniq_ts; but where times have gaps, ranks
+// leave hubs a group at (nearly) every key of their span, which the bucket tables
+// answer without a search.  Measured, ranks and offsets, 10M walks of 80 (T unique
+// timestamps, gap: time units per timestamp; ExponentialIndex over 20M edges):
+//  - every unit used (offsets are the ranks): T = 300k 15.6 and 15.1 ms;
+//  - lookups within an XCD's 4 MiB of L2: T = 500k, gap 1.5 16.7 and 17.7, T =
+//    300k, gap 2 15.6 and 17.5 (backward, 3M walks: 5.2 and 5.9);
+//  - past it: T = 550k, gap 1.5 23.5 and 17.9, T = 1M, gap 2 25.1 and 19.5;
+//  - T = 300k, gap 2 with weights (ExponentialWeight, 5M edges) 23.9 and 20.6;
+//  - with 50M edges, whose slot words have no room for a rank (the edge's
+//    timestamp is looked up) 29.2 and 24.5;
+//  - gap 10: T = 100k 13.7 and 16.5; T = 1M without room in the words
+//    (ExponentialWeight, 50M edges) 37.4 and 27.4.
+// So offsets where at most kTimeKeyGap units go to a timestamp and every unit
+// occurs, the lookup table is larger than kRankTableMax, the index has weights,
+// or a slot word cannot hold a rank.
 constexpr uint64_t kTimeKeyGap = 2;
+constexpr uint64_t kRankTableMax = 1ull << 19;
 constexpr uint64_t kTimeKeyMax = 0x7ffffff0ull;  // keys stay non-negative int32 values
 
 // Where node id, key and edge id do not fit in a 64-bit slot word together,

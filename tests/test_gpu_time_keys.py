@@ -50,6 +50,26 @@ def test_walks_on_offset_and_rank_keys(rule, t0, directed):
                    cutoffs=cuts, seed=3)
 
 
+@pytest.mark.parametrize("gap", [1, 2])
+@pytest.mark.parametrize("T", [1 << 19, (1 << 19) + 1])
+def test_index_walks_at_the_rank_tables_limit(T, gap):
+    """Without weights, gapped times are keyed by rank up to 2^19 unique
+    timestamps and by offset past them; gapless ones always by offset."""
+    rng = np.random.default_rng(27)
+    n = T + 1_000
+    units = gap * np.arange(T, dtype=np.int64) - 5_000
+    t = np.concatenate([units, rng.choice(units, n - T)])[rng.permutation(n)]
+    s, d, _ = graphs.powerlaw(3_000, n, s=1.4, seed=28)
+    og, eng = _pair(True, [(s, d, t)])
+    _assert_index_equal(og, eng)
+    for forward in (True, False):
+        _walk_case(og, eng, "ExponentialIndex", "Linear", forward, "total", 20, 2_000, seed=29)
+        seeds = np.unique(s[:100]).astype(np.int32)
+        cuts = rng.integers(units[0], units[-1] + 2, seeds.size)
+        _walk_case(og, eng, "Linear", "Uniform", forward, "nodes", 16, 3, seed_nodes=seeds,
+                   cutoffs=cuts, seed=30)
+
+
 @pytest.mark.parametrize("gap", [False, True])
 def test_weight_walks_on_key_blocks(gap):
     """22 + 22 + 22 bits do not fit a slot word: it holds 20 bits of the key's
