@@ -5,7 +5,7 @@ trw_sample_device for the same call -- on consecutive calls, the second
 smaller than the first, across start modes, processing orders, shuffles,
 cutoffs, replay draws, edge features and the weight pickers -- and every
 call runs with the engine's allocation hook armed, so any device allocation
-inside it would fail the call.  Calls of two handles from two threads take
+(or staging lane of the host copies) inside it would fail the call.  Calls of two handles from two threads take
 the device's array in turn.  Through the C ABI."""
 import numpy as np
 import pytest
@@ -73,7 +73,8 @@ def _noalloc(eng, cap, L, dim, mode, bias, n, **kw):
 
 def _call_noalloc(eng, cap, L, dim, mode, bias, n, bufs, **kw):
     """The call with the engine's allocation hook armed: the first device
-    allocation of any handle would fail it (MemoryError)."""
+    allocation (or staging lane taken) of any handle would fail it
+    (MemoryError)."""
     from temporal_random_walk import capi
     capi.debug_fail_allocation(0)
     try:
