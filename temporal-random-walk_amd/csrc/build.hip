@@ -1192,9 +1192,8 @@ __device__ __forceinline__ int heavy_tile_node(const uint32_t* tile_base, uint32
 // sums 16 consecutive groups; timestamps, group starts and weights move in rows
 // of 256 consecutive groups and change hands through LDS (a thread's run padded
 // by one value against bank conflicts), since a wave's access to 64 threads' runs
-// touches 64 lines for 512 bytes.  Bound by HBM then: with the global
-// weights' scans read the same way, an ingest of 20M weighted edges went from
-// 7.53 to 7.33 ms.
+// touches 64 lines for 512 bytes.  Bound by HBM then: 248 -> 170 us per launch
+// over 20M weighted edges.
 __global__ __launch_bounds__(256) void heavy_tile_scan_kernel(
     const uint32_t* __restrict__ heavy, const uint32_t* __restrict__ tile_base,
     const uint32_t* __restrict__ nh_dev, const uint32_t* __restrict__ cnt,
@@ -1268,7 +1267,9 @@ __global__ __launch_bounds__(256) void heavy_tile_scan_kernel(
 // forward): its tiles' exclusive prefixes, each the previous prefix plus the
 // previous tile's last value, so consecutive tiles stay non-decreasing across
 // their boundary; the node's total follows.  Bound by the chain of loads of the
-// largest node's tiles.
+// largest node's tiles: 39 us per launch over 20M weighted edges, 59 with one
+// thread for both directions.  (One loop of 32 loads, masked past the end, is
+// not kept in flight: 185 us; from clamped addresses 93.)
 __global__ void heavy_tile_prefix_kernel(const uint32_t* __restrict__ tile_base,
                                          const uint32_t* __restrict__ nh_dev,
                                          double* __restrict__ tsum_f, double* __restrict__ tsum_b,
@@ -1278,21 +1279,25 @@ __global__ void heavy_tile_prefix_kernel(const uint32_t* __restrict__ tile_base,
     if (i >= *nh_dev) return;
     double* ts = blockIdx.y == 0 ? tsum_b : tsum_f;
     double run = 0.0;
+    uint32_t t = tile_base[i];
     const uint32_t te = tile_base[i + 1];
-    // 32 tile sums are loaded before the running sum consumes them, so the
-    // loads are in flight together, the last batch's too; the additions keep
-    // tile order
-    constexpr uint32_t kBatch = 32;
-    for (uint32_t t = tile_base[i]; t < te; t += kBatch) {
+    // 16 tile sums are loaded before the running sum consumes them, so the
+    // loads are in flight together; the additions keep tile order
+    constexpr uint32_t kBatch = 16;
+    for (; t + kBatch <= te; t += kBatch) {
         double x[kBatch];
 #pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j) x[j] = j < te - t ? ts[t + j] : 0.0;
+        for (uint32_t j = 0; j < kBatch; ++j) x[j] = ts[t + j];
 #pragma unroll
         for (uint32_t j = 0; j < kBatch; ++j) {
-            if (j >= te - t) break;
             ts[t + j] = run;
             run = run + x[j];
         }
+    }
+    for (; t < te; ++t) {
+        const double x = ts[t];
+        ts[t] = run;
+        run = run + x;
     }
     (blockIdx.y == 0 ? total_b : total_f)[i] = run;
 }
