@@ -56,8 +56,9 @@ KERNEL_SOURCES = {
 
 
 # kernels of the walk path; every other kernel belongs to the index build
-WALK_PATH_KERNELS = ("walk_kernel", "walk_rows_kernel", "walk_start_kernel", "layout_",
-                     "walk_stats",
+WALK_PATH_KERNELS = ("walk_kernel", "walk_rows_kernel", "walk_start_", "layout_",
+                     "walk_stats", "flag_counts_kernel", "flag_ids_kernel", "mark_ids_kernel",
+                     "clear_bytes_kernel", "random_keys_kernel", "expand_starts_kernel",
                      "node_group_init", "node_group_segment", "gather_walk_features")
 
 
